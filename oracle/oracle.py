@@ -68,7 +68,7 @@ class RejectDiag(C.Structure):
 def build(ref: bool = True) -> None:
     """Compiles liboracle.so, and _ref/libref.so when the reference checkout is present."""
     subprocess.run(["make", "-s", "-C", HERE, "liboracle.so"], check=True)
-    if ref and os.path.isdir(os.environ.get("TWD_REFERENCE", "/root/reference")):
+    if ref and os.path.isfile(os.path.join(os.environ.get("TWD_REFERENCE", "/root/reference"), "src", "sampling.cpp")):
         subprocess.run(["make", "-s", "-C", HERE, "ref",
                         "REF=" + os.environ.get("TWD_REFERENCE", "/root/reference")], check=True)
 
