@@ -18,6 +18,7 @@
 #include <type_traits>
 #include <cstring>
 #include <string>
+#include <vector>
 
 #include "twd_internal.h"
 
@@ -45,11 +46,11 @@ struct HeadArgs {
     float softcap;
     float* logits;
     uint32_t vocab;
-    // greedy finish: running per-row maxima (zero between launches), the arrival counter
-    // {epoch, count} and this launch's epoch, and where the last block puts its results
-    uint64_t* gbest;    // [TWD_MAX_ROWS]
-    uint64_t* gctr;     // [kArriveWords]: grid_arrive's counter
-    uint32_t epoch, next_epoch;
+    // greedy finish: running per-row maxima of each group of blocks (zero between launches), the
+    // arrival counters and this launch's epoch, and where the last block puts its results
+    uint64_t* gbest;    // finish_max: [kFinGroups][TWD_MAX_ROWS]
+    uint64_t* gctr;     // [kFinCtrWords]: grid_arrive_tree's counters
+    FinishEpochs ep;
     uint32_t* tokens;
     const uint32_t* drafts;
     uint32_t n_drafts;
@@ -137,11 +138,18 @@ __device__ __forceinline__ bf16x8_t nibbles_to_bf16(uint32_t w, uint32_t magic) 
     return __builtin_bit_cast(bf16x8_t, p);
 }
 
+// Two floats to a bf16 pair (lo in the low half), round to nearest even: one instruction
+// (v_cvt_pk_bf16_f32) where f32_to_bf16_rne is about six per value. The same bits for every float
+// that is not a NaN; a NaN stays one.
+__device__ __forceinline__ uint32_t f32x2_to_bf16(float lo, float hi) {
+    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+    typedef float f32x2_t __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{lo, hi}), bf16x2_t));
+}
+
 // -h/128 of a bf16 pair, exact for every |h| >= 2^-119.
 __device__ __forceinline__ uint32_t neg_over_128(uint32_t v) {
-    const uint32_t lo = f32_to_bf16_rne(bf16_lo(v) * -0.0078125f);
-    const uint32_t hi = f32_to_bf16_rne(bf16_hi(v) * -0.0078125f);
-    return lo | (hi << 16);
+    return f32x2_to_bf16(bf16_lo(v) * -0.0078125f, bf16_hi(v) * -0.0078125f);
 }
 
 // One 16-byte slice of h (8 bf16 values e0..e7) as an A-fragment entry: permuted into the
@@ -176,50 +184,70 @@ __device__ __forceinline__ float sum8_bf16(u32x4_t v) {
 // bias_slices writes the four slice dwords of one (m, group) entry; at(kg) addresses them.
 template <typename At>
 __device__ __forceinline__ void bias_slices(float x, At at) {
-    const uint32_t hi = f32_to_bf16_rne(x);
-    const float r1 = x - __uint_as_float(hi << 16);  // exact
-    const uint32_t mid = f32_to_bf16_rne(r1);
-    const float r2 = r1 - __uint_as_float(mid << 16);  // exact
-    const uint32_t lo = f32_to_bf16_rne(r2);
-    *at(0) = hi * 0x10001u;
-    *at(1) = mid * 0x10001u;
-    *at(2) = lo * 0x10001u;
+    const uint32_t hi = f32x2_to_bf16(x, x);  // each slice twice, as the pair it is stored as
+    const float r1 = x - bf16_hi(hi);         // exact
+    const uint32_t mid = f32x2_to_bf16(r1, r1);
+    const float r2 = r1 - bf16_hi(mid);       // exact
+    *at(0) = hi;
+    *at(1) = mid;
+    *at(2) = f32x2_to_bf16(r2, r2);
     *at(3) = 0u;
 }
 
 // Shared memory of the head epilogue (cross-wave greedy reduction).
-template <int NW>
+template <int NW, int ROWS = TWD_MAX_ROWS>
 struct EpiSharedT {
-    uint64_t red[NW][TWD_MAX_ROWS];
-    uint64_t seen[TWD_MAX_ROWS];
-    uint32_t tok[TWD_MAX_ROWS];
+    static constexpr int kRows = ROWS;
+    static constexpr uint32_t kWaves = NW;
+    uint64_t red[NW][ROWS];
+    uint64_t seen[ROWS];
+    uint32_t tok[ROWS];
     int last;
 };
-using EpiShared = EpiSharedT<kHeadWaves>;
 
 // Softcap, logits store, and -- for the greedy modes -- the per-row rank maximum over the
 // whole grid, finished by the last block to arrive (tokens, then greedy verify bookkeeping).
 //
-// Cross-block publication uses device-scope atomics only: each block folds its ranks into
-// gbest[m] with a returning atomic max, then counts itself in on the arrival counter; the block
-// that completes the count reads and clears gbest with atomic exchanges. Returning atomics are
+// Cross-block publication uses device-scope atomics only: each block folds its ranks into its
+// group's maxima with a returning atomic max, then counts itself in on the arrival counters; the
+// block that completes the count reads and clears the maxima with atomic exchanges. Returning atomics are
 // performed at the memory-side coherence point before they return, so every block's maxima
 // precede its arrival, and the last block observes all of them. No data travels through plain
 // stores, so no device-scope fence is needed: on this part such a fence writes back the XCD's
 // L2 and, paid by each of ~1000 blocks, costs more than the streaming pass itself.
 //
-// Arrivals are counted by grid_arrive on gctr (an epoch per launch, armed by the previous
+// Arrivals are counted by grid_arrive_tree on gctr (an epoch per launch, armed by the previous
 // launch's last block; replays of a captured launch count in on a replay slot, and only a launch
-// that finds neither armed for it pays for contended compare-and-swap retries).
+// that finds neither armed for it pays for contended compare-and-swap retries). Small heads' blocks
+// finish together and are spread over kFinGroups maxima and counters, because atomics on one
+// address are served one by one: with one of each, a greedy launch took 3.8 us longer than the
+// same launch without its finish on 251 blocks (V = 32,003, d = 2,048; 12.3 against 8.5 us),
+// spread 2.3 us. Where the blocks finish apart (one block per CU with two or more tiles per wave,
+// and the wide kernels) the second level only costs its round trip (V = 262,144: M = 12 139.8
+// against 137.7 us, M = 5 126.5 against 125.4).
 // tot[j][mt][i] holds row r = (tile0 + j) * 16 + lane % 16 of MFMA row 16 mt + 4 (lane / 16) + i,
 // which carries h row m = (16 mt + 4 (lane / 16) + i) / MS when i is a multiple of MS (MS > 1:
 // the rows are spread over the MFMA rows, see head_small_kernel); other entries are not outputs.
-template <int NW>
-__device__ __forceinline__ void grid_finish(const HeadArgs& a, EpiSharedT<NW>& se);
+template <typename Epi>
+__device__ __forceinline__ void grid_finish(const HeadArgs& a, Epi& se);
 
-template <int NMT, int NI, int RT, int MODE, int NW, int MS = 1>
+// The maximum over the 16 lanes of a row of lanes, in each of them: DPP quad_perm [1,0,3,2] and
+// [2,3,0,1], row_half_mirror, row_mirror. A row's 16 lanes are active together.
+__device__ __forceinline__ uint64_t row16_max_u64(uint64_t k) {
+    auto step = [&](auto ctrl) {
+        const uint64_t o = dpp_move<decltype(ctrl)::value>(k, k);
+        k = o > k ? o : k;
+    };
+    step(std::integral_constant<int, 0xB1>{});
+    step(std::integral_constant<int, 0x4E>{});
+    step(std::integral_constant<int, 0x141>{});
+    step(std::integral_constant<int, 0x140>{});
+    return k;
+}
+
+template <int NMT, int NI, int RT, int MODE, int MS = 1, typename Epi>
 __device__ __forceinline__ void head_epilogue(const HeadArgs& a, f32x4_t (&tot)[RT][NMT],
-                                              uint32_t tile0, EpiSharedT<NW>& se) {
+                                              uint32_t tile0, Epi& se) {
     static_assert(MS == 1 || (NMT == 1 && NI == 4), "spread rows live in one m tile");
     if (NMT == 1 && a.fold) {  // rows r and r + 8 sit in lanes l and l + 32
 #pragma unroll
@@ -254,59 +282,76 @@ __device__ __forceinline__ void head_epilogue(const HeadArgs& a, f32x4_t (&tot)[
     }
     if (MODE == kModeLogits) return;
 
-    // rows sharing m are the 16 lanes with the same lane >> 4, one DPP row: quad_perm [1,0,3,2]
-    // and [2,3,0,1], row_half_mirror, row_mirror (register moves, where a shuffle is an LDS
-    // round trip at the end of every wave)
+    // rows sharing m are the 16 lanes with the same lane >> 4, one DPP row (register moves, where a
+    // shuffle is an LDS round trip at the end of every wave)
 #pragma unroll
     for (int mt = 0; mt < NMT; ++mt)
 #pragma unroll
         for (int i = 0; i < NI; i += MS) {
-            uint64_t k = best[mt][i];
-            auto step = [&](auto ctrl) {
-                const uint64_t o = dpp_move<decltype(ctrl)::value>(k, k);
-                k = o > k ? o : k;
-            };
-            step(std::integral_constant<int, 0xB1>{});
-            step(std::integral_constant<int, 0x4E>{});
-            step(std::integral_constant<int, 0x141>{});
-            step(std::integral_constant<int, 0x140>{});
+            const uint64_t k = row16_max_u64(best[mt][i]);
             const uint32_t m = (mt * 16 + 4 * (lane >> 4) + i) / MS;
-            if ((lane & 15) == 0 && m < TWD_MAX_ROWS) se.red[wave][m] = k;
+            if ((lane & 15) == 0 && m < static_cast<uint32_t>(Epi::kRows)) se.red[wave][m] = k;
         }
-    grid_finish<NW>(a, se);
+    grid_finish(a, se);
 }
 
+// The running maxima of a group of blocks, [TWD_MAX_ROWS] each: group 0's at the start of the
+// finish state, the others' past the arrival counters.
+__host__ __device__ constexpr uint32_t finish_max(uint32_t group) {
+    return group == 0 ? 0u : TWD_MAX_ROWS * group + kFinCtrWords;
+}
+constexpr uint32_t kFinishWords = TWD_MAX_ROWS * kFinGroups + kFinCtrWords;
+
 // The greedy finish shared by the head kernels, once every wave has written its per-row maxima
-// to se.red[wave][m]: the block's maxima go to gbest, the block counts itself in, and the last
-// block of the launch writes the tokens (and the greedy verify bookkeeping).
-template <int NW>
-__device__ __forceinline__ void grid_finish(const HeadArgs& a, EpiSharedT<NW>& se) {
+// to se.red[wave][m]: the block's maxima go to its group's, the block counts itself in, and the
+// last block of the launch writes the tokens (and the greedy verify bookkeeping).
+template <typename Epi>
+__device__ __forceinline__ void grid_finish(const HeadArgs& a, Epi& se) {
     const int tid = threadIdx.x;
+    const uint32_t nw = blockDim.x >> 6;
     __syncthreads();
     const uint32_t nb = gridDim.x;
+    uint64_t* best = a.gbest + finish_max(finish_group(a.ep, blockIdx.x));
     if (static_cast<uint32_t>(tid) < a.M) {
-        uint64_t k = se.red[0][tid];
+        // eight waves' maxima requested together (of waves past the block's: not written, not used)
+        uint64_t k = 0;
+        for (uint32_t w0 = 0; w0 < nw; w0 += 8) {
 #pragma unroll
-        for (int w = 1; w < NW; ++w) k = se.red[w][tid] > k ? se.red[w][tid] : k;
+            for (uint32_t w = w0; w < w0 + 8; ++w) {
+                const uint64_t o = se.red[min(w, Epi::kWaves - 1)][tid];
+                k = w < nw && o > k ? o : k;
+            }
+        }
         // the returning form: the maximum is performed before this block counts itself in
-        se.seen[tid] = __hip_atomic_fetch_max(reinterpret_cast<unsigned long long*>(a.gbest + tid),
+        se.seen[tid] = __hip_atomic_fetch_max(reinterpret_cast<unsigned long long*>(best + tid),
                                               static_cast<unsigned long long>(k), __ATOMIC_RELAXED,
                                               __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
     if (tid == 0) {
-        const bool last = grid_arrive(reinterpret_cast<unsigned long long*>(a.gctr), nb, a.epoch, a.next_epoch);
-        se.last = last;
+        se.last = grid_arrive_tree(reinterpret_cast<unsigned long long*>(a.gctr), blockIdx.x, nb, a.ep);
     }
     __syncthreads();
     if (!se.last) return;
     // every other block's maximum was performed before its arrival was counted
-    if (static_cast<uint32_t>(tid) < a.M) {
-        const uint64_t k = __hip_atomic_exchange(reinterpret_cast<unsigned long long*>(a.gbest + tid),
-                                                 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    auto take = [&](uint32_t group, uint32_t m) -> uint64_t {
+        return __hip_atomic_exchange(reinterpret_cast<unsigned long long*>(a.gbest + finish_max(group) + m), 0ull,
+                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    auto put = [&](uint32_t m, uint64_t k) {
         const uint32_t t = rank_index(k);
-        se.tok[tid] = t;
-        if (a.tokens) a.tokens[tid] = t;
+        se.tok[m] = t;
+        if (a.tokens) a.tokens[m] = t;
+    };
+    if (a.ep.tree_epoch != 0) {
+        // the 16 lanes of a row of lanes read the groups' maxima of one row m
+        static_assert(kFinGroups == 16, "one group per lane of a row of lanes");
+        for (uint32_t m = static_cast<uint32_t>(tid) >> 4; m < a.M; m += blockDim.x >> 4) {
+            const uint64_t k = row16_max_u64(take(tid & 15, m));
+            if ((tid & 15) == 0) put(m, k);
+        }
+    } else if (static_cast<uint32_t>(tid) < a.M) {
+        put(tid, take(0, tid));
     }
     __syncthreads();
     if (tid < 64 && a.vres) verify_bookkeeping(se.tok, a.M, a.drafts, a.n_drafts, a.vres);
@@ -317,17 +362,17 @@ __device__ __forceinline__ void grid_finish(const HeadArgs& a, EpiSharedT<NW>& s
 // and 2g + 1 are entries 0 and 2 of lanes 16g .. 16g + 15. Per live entry: the softcap, then
 // apply_repetition_penalty (sampling.cpp:74-90) with the entry's occurrence count from the
 // block's LDS counts, one occurrence at a time (divide or multiply, then clamp), then the store.
-// Each wave then publishes, per row, the statistics of its 64 vocabulary rows that
+// Each wave then publishes, per row, the statistics of its 16 RT vocabulary rows that
 // select_sample_merge_kernel needs -- its best rank (value desc, index asc) and the sum of
 // exp(v - that value) in double, NaN when the wave saw a NaN (the row is then degenerate, as a
 // NaN makes the reference's total NaN) -- with no barrier and no cross-wave step. tbl holds
 // 2^(j/64), j < 64, for exp_for_sum.
-template <int RT, int NW, int MS>
+template <int RT, int MS>
 __device__ __forceinline__ void head_epilogue_sample(const HeadArgs& a, f32x4_t (&tot)[RT][1],
                                                      uint32_t tile0, uint32_t block_row0,
                                                      const uint32_t* cnt, const double* tbl,
                                                      const float* prm) {
-    constexpr uint32_t kRowsPerBlock = NW * RT * kTileRows;
+    const uint32_t nw = blockDim.x >> 6, block_rows = nw * RT * kTileRows;
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int e = 0; e < 4 / MS; ++e) {  // entry MS * e: h row (4 (lane / 16) + MS * e) / MS
@@ -345,7 +390,7 @@ __device__ __forceinline__ void head_epilogue_sample(const HeadArgs& a, f32x4_t 
             float x = tot[j][0][MS * e];
             if (a.softcap > 0.0f) x = a.softcap * tanhf(x / a.softcap);
             if (live && rp != 1.0f) {
-                const uint32_t n = cnt[mm * kRowsPerBlock + (r - block_row0)];
+                const uint32_t n = cnt[mm * block_rows + (r - block_row0)];
                 for (uint32_t t = 0; t < n; ++t) {
                     x = (x > 0.0f) ? (x / rp) : (x * rp);
                     if (lim > 0.0f) x = (x < -lim) ? -lim : ((lim < x) ? lim : x);
@@ -392,7 +437,7 @@ __device__ __forceinline__ void head_epilogue_sample(const HeadArgs& a, f32x4_t 
         for (int msk = 1; msk < 16; msk <<= 1) sum += __shfl_xor(sum, msk);
         if (nan) sum = __builtin_nan("");
         if ((lane & 15) == 0 && mlive) {
-            const size_t o = static_cast<size_t>(m) * (gridDim.x * NW) + blockIdx.x * NW + (threadIdx.x >> 6);
+            const size_t o = static_cast<size_t>(m) * (gridDim.x * nw) + blockIdx.x * nw + (threadIdx.x >> 6);
             a.stats.key[o] = best;
             a.stats.sum[o] = sum;
             a.stats.max[o] = nan ? __builtin_nanf("") : wm;
@@ -465,49 +510,58 @@ __device__ __forceinline__ uint32_t wave_id() {
     return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 }
 
-// ---- M <= 8: the whole h resident in LDS, no barrier in the streaming loop ---------------------
+// ---- M <= 16: the whole h resident in LDS, no barrier in the streaming loop --------------------
 //
 // LDS holds the prepared h in A-fragment order, [m][chunk U][k-step t][kg] of 16 B, and the bias
 // A-fragment entries [super-unit P][slice kg][m] of 16 B, both over npad = nunits rounded up to
-// the ring depth PF; the chunks past nunits hold zeros, so the streaming loop runs whole ring
-// cycles with no branch: its weight loads are clamped to the last unit, whose contribution the
-// zero h and zero bias entries cancel exactly (the loader rejects infinite biases and scales
-// above 2^100, so every product with those zeros is zero). A-fragment rows m >= M only feed
-// output rows that are never stored, so their lanes simply read row 0. Each wave streams its
-// RT row tiles through the PF-deep register ring with no synchronisation until the epilogue.
-template <int PF>
-__host__ __device__ constexpr uint32_t small_pad_units(uint32_t nunits) {
-    return (nunits + PF - 1) / PF * PF;
-}
+// whole super-units; an odd chunk count's last chunk holds zeros, and its weight loads re-read
+// the last unit, whose contribution the zero h and zero bias entries cancel exactly (the loader
+// rejects infinite biases and scales above 2^100, so every product with those zeros is zero).
+// A-fragment rows m >= M only feed output rows that are never stored, so their lanes simply read
+// row 0. Each wave streams its RT row tiles through the PF-deep register ring with no
+// synchronisation until the epilogue; the loop runs whole ring cycles with no branch (loads past
+// the last unit are clamped to it), and only the last cycle, which requests nothing, leaves out
+// the super-units past npad.
+__host__ __device__ constexpr uint32_t resident_pad_units(uint32_t nunits) { return (nunits + 1) & ~1u; }
 
 //
 // MS spreads the rows over the MFMA's 16 A rows: h row m sits in A row MS * m, so its outputs
 // land in accumulator entry i = (MS * m) % 4 of the lanes with lane / 16 = MS * m / 4. With
 // MS = 4 (M <= 4) every output is entry 0 and each group costs one scale FMA per accumulator
-// instead of four; MS = 2 (M <= 8) uses entries 0 and 2. A rows that carry no h row read row 0;
-// their outputs are never stored.
+// instead of four; MS = 2 (M <= 8) uses entries 0 and 2, MS = 1 (M <= 16) all four. A rows that
+// carry no h row read row 0; their outputs are never stored.
 //
-// NORM: the final RMSNorm as the prologue (M <= 4). Each block computes the rows' mean squares
-// itself and stages h = (x * rms) * w, which is fp32, as two bf16 halves hi = bf16(h) and
-// lo = bf16(h - hi) (|h - hi - lo| <= 2^-18 |h|) in LDS rows 2m and 2m + 1, fed as A rows 4m
-// and 4m + 1; their outputs, entries 0 and 1 of one lane, are added before the softcap. The
-// bias term uses the group sums of hi + lo (what the MFMA rows carry), on the hi rows only.
-template <int MS, int RT, int PF, int NW, int MODE, bool NORM = false>
-__global__ __launch_bounds__(NW * 64) void head_small_kernel(HeadArgs a) {
+// NORM: the final RMSNorm as the prologue (M <= 4 with MS = 4, M <= 8 with MS = 2). Each block
+// computes the rows' mean squares itself and stages h = (x * rms) * w, which is fp32, as two bf16
+// halves hi = bf16(h) and lo = bf16(h - hi) (|h - hi - lo| <= 2^-18 |h|) in LDS rows 2m and
+// 2m + 1, fed as A rows MS m and MS m + 1; their outputs, adjacent entries of one lane, are added
+// before the softcap. The bias term uses the group sums of hi + lo (what the MFMA rows carry), on
+// the hi rows only.
+//
+// A block has blockDim.x / 64 <= NWM waves and owns that many times RT row tiles (resident_shape
+// picks RT and the waves).
+// Deepest head: 66 chunks, 8 rows of which fit in LDS beside the finish state.
+constexpr int kResidentWaves = 16;
+constexpr uint32_t kMaxUnits = 66;
+constexpr int kResidentRows = 16;
+
+template <int MS, int RT, int PF, int MODE, bool NORM = false>
+__global__ __launch_bounds__(kResidentWaves * 64) void head_small_kernel(HeadArgs a) {
     static_assert(PF % 2 == 0, "the ring holds whole super-units");
-    static_assert(MS == 2 || MS == 4, "rows spread over 16 MFMA rows with stride 2 or 4");
-    static_assert(!NORM || MS == 4, "the RMSNorm prologue takes two MFMA rows per h row");
-    constexpr int NT = NW * 64;
+    static_assert(MS == 1 || MS == 2 || MS == 4, "rows spread over 16 MFMA rows with stride 1, 2 or 4");
+    static_assert(!NORM || MS >= 2, "the RMSNorm prologue takes two MFMA rows per h row");
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    __shared__ EpiSharedT<NW> se;
+    __shared__ EpiSharedT<kResidentWaves, kResidentRows> se;
+    const uint32_t nw = __builtin_amdgcn_readfirstlane(blockDim.x >> 6);
+    const uint32_t NT = nw * 64;
     u32x4_t* sH = reinterpret_cast<u32x4_t*>(smem_raw);
     const uint32_t row_vecs = a.d / 8;  // 16 B vectors per h row
-    const uint32_t npad = small_pad_units<PF>(a.nunits);
+    const uint32_t npad = resident_pad_units(a.nunits);
     const uint32_t pad_vecs = npad * 16;  // 16 B vectors per padded LDS row
     const uint32_t lrows = NORM ? 2 * a.M : a.M;  // LDS rows of prepared h
     u32x4_t* sXF = sH + lrows * pad_vecs;          // [super-units][4][lrows]
-    const int tid = threadIdx.x, lane = tid & 63;
-    const uint32_t tile0 = (blockIdx.x * NW + wave_id()) * RT;
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t tile0 = (blockIdx.x * nw + wave_id()) * RT;
     const uint32_t magic = vgpr_const(0x43004300u);
 
     __amdgpu_buffer_rsrc_t rs[RT];
@@ -516,19 +570,20 @@ __global__ __launch_bounds__(NW * 64) void head_small_kernel(HeadArgs a) {
     const uint32_t last = a.nunits - 1;
     u32x4_t wq[PF][RT];
     u32x2_t sq[PF][RT];
-    // sample mode: occurrence counts of the block's rows in each row's history (16 / MS rows)
-    constexpr uint32_t kRowsPerBlock = NW * RT * kTileRows;
+    // sample mode: occurrence counts of the block's rows in each row's history (16 / MS rows),
+    // past the staged h
+    const uint32_t block_rows = nw * RT * kTileRows;
     constexpr uint32_t kCntRows = 16 / MS;
-    __shared__ uint32_t cnt[MODE == kModeSample ? kCntRows * kRowsPerBlock : 1];
+    uint32_t* cnt = reinterpret_cast<uint32_t*>(sXF + npad * 2 * lrows);
     __shared__ double exp2_tbl[MODE == kModeSample ? 64 : 1];
     // the rows' penalty factors and clamps, read per lane in the epilogue: staged here, where the
     // load overlaps the ring fill, instead of a memory round trip at the end of every block
     __shared__ float prm[MODE == kModeSample ? 3 * kSampleRows : 1];
-    const uint32_t block_row0 = blockIdx.x * kRowsPerBlock;
+    const uint32_t block_row0 = blockIdx.x * block_rows;
     if constexpr (MODE == kModeSample) {
-        for (uint32_t i = tid; i < kCntRows * kRowsPerBlock; i += NT) cnt[i] = 0;
-        if (tid < 64) exp2_tbl[tid] = kExp2Table[tid];
-        if (tid < static_cast<int>(kSampleRows)) {
+        for (uint32_t i = tid; i < kCntRows * block_rows; i += NT) cnt[i] = 0;
+        for (uint32_t i = tid; i < 64; i += NT) exp2_tbl[i] = kExp2Table[i];
+        if (tid < kSampleRows) {
             prm[tid] = a.rp[tid];
             prm[kSampleRows + tid] = a.clamp[tid];
             prm[2 * kSampleRows + tid] = a.ref[tid];
@@ -556,11 +611,53 @@ __global__ __launch_bounds__(NW * 64) void head_small_kernel(HeadArgs a) {
         }
     }
 
-    // The ring is filled before h is staged, so the two memory round trips overlap. Ring order,
-    // the same in the prologue and in every cycle: per super-unit, the even unit's nibbles, then
-    // its {b, t} words, then the odd unit's nibbles and words. The even unit's words are refilled
-    // only after the odd step's bias MFMA has read them, so the bias fragment needs no copy that
-    // outlives the refill.
+    // One or two tiles per wave: the first rows of h are requested before the ring is filled.
+    // Loads complete in order, so the staging below then waits for h alone while the ring's first
+    // units are still on their way from HBM. Four tiles per wave (large heads, where the fill is a
+    // small part) measured faster the other way round: 116.4 against 117.8 us (M = 1 logits,
+    // V = 262,144, d = 5,376).
+    constexpr int kBatch = 4;
+    const uint32_t tasks = a.M * pad_vecs;
+    u32x4_t hv[NORM ? 1 : kBatch];
+    auto load_h = [&](uint32_t base) {
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b) {
+            const uint32_t task = base + b * NT + tid;
+            const uint32_t m = task / pad_vecs, c8 = task % pad_vecs;
+            hv[b] = u32x4_t{0u, 0u, 0u, 0u};
+            if (task < tasks && c8 < row_vecs)
+                hv[b] = *reinterpret_cast<const u32x4_t*>(a.h + (static_cast<size_t>(m) * row_vecs + c8) * 8);
+        }
+    };
+    // NORM: a vector of x and of the weight (one per thread and step)
+    struct XVec {
+        float4 x0, x1;
+        u32x4_t w;
+    };
+    auto load_x = [&](uint32_t task) {
+        XVec r{float4{0.f, 0.f, 0.f, 0.f}, float4{0.f, 0.f, 0.f, 0.f}, u32x4_t{0u, 0u, 0u, 0u}};
+        const uint32_t m = task / pad_vecs, c8 = task % pad_vecs;
+        if (task < tasks && c8 < row_vecs) {
+            const float* xrow = a.x + static_cast<size_t>(m) * a.d + c8 * 8;
+            r.x0 = *reinterpret_cast<const float4*>(xrow);
+            r.x1 = *reinterpret_cast<const float4*>(xrow + 4);
+            r.w = *reinterpret_cast<const u32x4_t*>(a.norm_w + c8 * 8);
+        }
+        return r;
+    };
+    XVec xv{};
+    auto first_h = [&]() {
+        if constexpr (NORM)
+            xv = load_x(tid);
+        else
+            load_h(0);
+    };
+    if constexpr (RT < 4 || NORM) first_h();
+
+    // Ring order, the same in the prologue and in every cycle: per super-unit, the even unit's
+    // nibbles, then its {b, t} words, then the odd unit's nibbles and words. The even unit's
+    // words are refilled only after the odd step's bias MFMA has read them, so the bias fragment
+    // needs no copy that outlives the refill.
 #pragma unroll
     for (int s = 0; s < PF; ++s) {
         const uint32_t U = min(static_cast<uint32_t>(s), last);
@@ -568,109 +665,79 @@ __global__ __launch_bounds__(NW * 64) void head_small_kernel(HeadArgs a) {
         load_scales_ordered<RT>(rs, U, vo_s, sq[s]);
     }
 
+    if constexpr (!(RT < 4 || NORM)) first_h();
     // ---- stage h: 8 consecutive threads cover one 64-column group; padding chunks get zeros.
     // Each thread issues kBatch loads before it waits, so a block pays about one round trip per
     // kBatch * NT vectors.
-    constexpr int kBatch = 4;
-    const uint32_t tasks = a.M * pad_vecs;
     // NORM: the per-row scale 1 / sqrt(mean(x^2) + eps) is common to every term of a row's
     // logit, so h' = x * w is staged and the sum is scaled once in the epilogue; the mean
-    // squares are gathered from the same loads (partial sums per wave in ss_red).
-    __shared__ float ss_red[NORM ? NW : 1][4];
+    // squares are gathered from the same loads (partial sums per super-unit in ss_red).
+    __shared__ float ss_red[NORM ? kMaxUnits / 2 * (16 / MS) : 1];
     if constexpr (NORM) {
-        // row by row, so each thread's square sum belongs to one row; one vector per thread in
-        // flight (its temporaries share the registers with the filled weight ring: two would
-        // cost a wave per SIMD)
-        constexpr int kBatchN = 1;
+        // the next vector is requested before this one is used
         uint32_t* xo = reinterpret_cast<uint32_t*>(sXF);
-        for (uint32_t m = 0; m < a.M; ++m) {
-            const float* xrow = a.x + static_cast<size_t>(m) * a.d;
-            float ssm = 0.0f;
-            for (uint32_t base = 0; base < pad_vecs; base += NT * kBatchN) {
-                float4 x0[kBatchN], x1[kBatchN];
-                u32x4_t wv[kBatchN];
+        for (uint32_t base = 0; base < tasks; base += NT) {
+            const uint32_t task = base + tid;
+            const XVec cur = xv;
+            xv = load_x(task + NT);
+            const float xs[8] = {cur.x0.x, cur.x0.y, cur.x0.z, cur.x0.w, cur.x1.x, cur.x1.y, cur.x1.z, cur.x1.w};
+            const uint32_t ws[4] = {cur.w.x, cur.w.y, cur.w.z, cur.w.w};
+            u32x4_t vh, vl;
+            float sum = 0.0f, ssm = 0.0f;
 #pragma unroll
-                for (int b = 0; b < kBatchN; ++b) {
-                    const uint32_t c8 = base + b * NT + tid;
-                    x0[b] = x1[b] = float4{0.f, 0.f, 0.f, 0.f};
-                    wv[b] = u32x4_t{0u, 0u, 0u, 0u};
-                    if (c8 < row_vecs) {
-                        x0[b] = *reinterpret_cast<const float4*>(xrow + c8 * 8);
-                        x1[b] = *reinterpret_cast<const float4*>(xrow + c8 * 8 + 4);
-                        wv[b] = *reinterpret_cast<const u32x4_t*>(a.norm_w + c8 * 8);
-                    }
-                }
-#pragma unroll
-                for (int b = 0; b < kBatchN; ++b) {
-                    const uint32_t c8 = base + b * NT + tid;
-                    const float xs[8] = {x0[b].x, x0[b].y, x0[b].z, x0[b].w, x1[b].x, x1[b].y, x1[b].z, x1[b].w};
-                    const uint32_t ws[4] = {wv[b].x, wv[b].y, wv[b].z, wv[b].w};
-                    uint32_t hi[8], lo[8];
-                    float sum = 0.0f;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const uint32_t wb = (ws[e >> 1] >> (16 * (e & 1))) & 0xFFFFu;
-                        const float he = xs[e] * __uint_as_float(wb << 16);  // x * weight
-                        hi[e] = f32_to_bf16_rne(he);
-                        lo[e] = f32_to_bf16_rne(he - __uint_as_float(hi[e] << 16));
-                        // the sum of what the MFMA rows carry (hi + lo, exact in fp32), so that
-                        // the bias term cancels their 128 X exactly
-                        sum += __uint_as_float(hi[e] << 16) + __uint_as_float(lo[e] << 16);
-                        ssm += xs[e] * xs[e];
-                    }
-                    sum += __shfl_xor(sum, 1);
-                    sum += __shfl_xor(sum, 2);
-                    sum += __shfl_xor(sum, 4);
-                    if (c8 < pad_vecs) {
-                        const uint32_t U = c8 >> 4, c = c8 & 15;
-                        const u32x4_t vh = u32x4_t{hi[0] | (hi[1] << 16), hi[2] | (hi[3] << 16),
-                                                   hi[4] | (hi[5] << 16), hi[6] | (hi[7] << 16)};
-                        const u32x4_t vl = u32x4_t{lo[0] | (lo[1] << 16), lo[2] | (lo[3] << 16),
-                                                   lo[4] | (lo[5] << 16), lo[6] | (lo[7] << 16)};
-                        sH[(((2 * m) * npad + U) * 4 + (c >> 2)) * 4 + (c & 3)] = prep_h(vh);
-                        sH[(((2 * m + 1) * npad + U) * 4 + (c >> 2)) * 4 + (c & 3)] = prep_h(vl);
-                        if ((c8 & 7) == 0) {
-                            const uint32_t g = c8 >> 3;
-                            bias_slices(sum, [&](int kg) {
-                                return xo + (((g >> 2) * 4 + kg) * lrows + 2 * m) * 4 + (g & 3);
-                            });
-                            bias_slices(0.0f, [&](int kg) {
-                                return xo + (((g >> 2) * 4 + kg) * lrows + 2 * m + 1) * 4 + (g & 3);
-                            });
-                        }
-                    }
-                }
+            for (int e = 0; e < 4; ++e) {
+                const float h0 = xs[2 * e] * bf16_lo(ws[e]), h1 = xs[2 * e + 1] * bf16_hi(ws[e]);  // x * weight
+                vh[e] = f32x2_to_bf16(h0, h1);
+                vl[e] = f32x2_to_bf16(h0 - bf16_lo(vh[e]), h1 - bf16_hi(vh[e]));
+                // the sum of what the MFMA rows carry (hi + lo, exact in fp32), so that
+                // the bias term cancels their 128 X exactly
+                sum += bf16_lo(vh[e]) + bf16_lo(vl[e]);
+                sum += bf16_hi(vh[e]) + bf16_hi(vl[e]);
+                ssm += xs[2 * e] * xs[2 * e];
+                ssm += xs[2 * e + 1] * xs[2 * e + 1];
             }
+            sum += __shfl_xor(sum, 1);
+            sum += __shfl_xor(sum, 2);
+            sum += __shfl_xor(sum, 4);
+            // a super-unit's 32 vectors are half a wave (a row holds whole super-units)
 #pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) ssm += __shfl_xor(ssm, o);
-            if (lane == 0) ss_red[tid >> 6][m] = ssm;
-        }
-    } else
-    for (uint32_t base = 0; base < tasks; base += NT * kBatch) {
-        u32x4_t v[kBatch];
-#pragma unroll
-        for (int b = 0; b < kBatch; ++b) {
-            const uint32_t task = base + b * NT + tid;
-            const uint32_t m = task / pad_vecs, c8 = task % pad_vecs;
-            v[b] = u32x4_t{0u, 0u, 0u, 0u};
-            if (task < tasks && c8 < row_vecs)
-                v[b] = *reinterpret_cast<const u32x4_t*>(a.h + (static_cast<size_t>(m) * row_vecs + c8) * 8);
-        }
-#pragma unroll
-        for (int b = 0; b < kBatch; ++b) {
-            const uint32_t task = base + b * NT + tid;
-            const uint32_t m = task / pad_vecs, c8 = task % pad_vecs;
-            float s = sum8_bf16(v[b]);
-            s += __shfl_xor(s, 1);
-            s += __shfl_xor(s, 2);
-            s += __shfl_xor(s, 4);
+            for (int o = 1; o < 32; o <<= 1) ssm += __shfl_xor(ssm, o);
             if (task < tasks) {
+                const uint32_t m = task / pad_vecs, c8 = task % pad_vecs;
                 const uint32_t U = c8 >> 4, c = c8 & 15;
-                sH[((m * npad + U) * 4 + (c >> 2)) * 4 + (c & 3)] = prep_h(v[b]);
+                sH[(((2 * m) * npad + U) * 4 + (c >> 2)) * 4 + (c & 3)] = prep_h(vh);
+                sH[(((2 * m + 1) * npad + U) * 4 + (c >> 2)) * 4 + (c & 3)] = prep_h(vl);
                 if ((c8 & 7) == 0) {
                     const uint32_t g = c8 >> 3;
-                    uint32_t* x = reinterpret_cast<uint32_t*>(sXF);
-                    bias_slices(s, [&](int kg) { return x + (((g >> 2) * 4 + kg) * a.M + m) * 4 + (g & 3); });
+                    bias_slices(sum, [&](int kg) {
+                        return xo + (((g >> 2) * 4 + kg) * lrows + 2 * m) * 4 + (g & 3);
+                    });
+                    bias_slices(0.0f, [&](int kg) {
+                        return xo + (((g >> 2) * 4 + kg) * lrows + 2 * m + 1) * 4 + (g & 3);
+                    });
+                }
+                if ((c8 & 31) == 0) ss_red[task / 32] = ssm;  // row m's super-unit c8 / 32
+            }
+        }
+    } else {
+        for (uint32_t base = 0; base < tasks; base += NT * kBatch) {
+            if (base != 0) load_h(base);
+#pragma unroll
+            for (int b = 0; b < kBatch; ++b) {
+                const uint32_t task = base + b * NT + tid;
+                const uint32_t m = task / pad_vecs, c8 = task % pad_vecs;
+                float s = sum8_bf16(hv[b]);
+                s += __shfl_xor(s, 1);
+                s += __shfl_xor(s, 2);
+                s += __shfl_xor(s, 4);
+                if (task < tasks) {
+                    const uint32_t U = c8 >> 4, c = c8 & 15;
+                    sH[((m * npad + U) * 4 + (c >> 2)) * 4 + (c & 3)] = prep_h(hv[b]);
+                    if ((c8 & 7) == 0) {
+                        const uint32_t g = c8 >> 3;
+                        uint32_t* x = reinterpret_cast<uint32_t*>(sXF);
+                        bias_slices(s, [&](int kg) { return x + (((g >> 2) * 4 + kg) * a.M + m) * 4 + (g & 3); });
+                    }
                 }
             }
         }
@@ -683,7 +750,7 @@ __global__ __launch_bounds__(NW * 64) void head_small_kernel(HeadArgs a) {
 #pragma unroll
             for (int q = 0; q < kHistBatch; ++q) {
                 const uint32_t lr = ids[q] - block_row0;
-                if (lr < kRowsPerBlock) atomicAdd(&cnt[m * kRowsPerBlock + lr], 1u);
+                if (lr < block_rows) atomicAdd(&cnt[m * block_rows + lr], 1u);
             }
         };
         if (m_first < a.M) count(m_first, hids);
@@ -712,13 +779,9 @@ __global__ __launch_bounds__(NW * 64) void head_small_kernel(HeadArgs a) {
     const u32x4_t* aRow = sH + lrow * pad_vecs + (lane >> 4);
     const u32x4_t* xRow = sXF + (lane >> 4) * lrows + lrow;
 
-    f32x4_t tot[RT][1], bacc[RT];
+    f32x4_t tot[RT][1];
 #pragma unroll
-    for (int j = 0; j < RT; ++j) {
-        tot[j][0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        bacc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    }
-
+    for (int j = 0; j < RT; ++j) tot[j][0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
     // One unit of the ring: slot s holds chunk U0 + s; RELOAD refills the slot PF chunks ahead.
     auto step = [&](uint32_t U0, auto slot, auto reload) {
@@ -755,13 +818,21 @@ __global__ __launch_bounds__(NW * 64) void head_small_kernel(HeadArgs a) {
         if constexpr ((s & 1) == 0) {
             if constexpr (kReload) load_nibbles_ordered<RT>(rs, Un, vo_w, wq[s]);
         } else {
-            // {b, t} words of the super-unit's four groups: the bias B fragment
+            // {b, t} words of the super-unit's four groups: the bias B fragment. The bias is added
+            // super-unit by super-unit: it cancels the 128 X that the groups' FMAs bring, so the
+            // running sum stays of the logit's own size (summed apart to the end, both parts grow
+            // some 17 times larger, and the logits of V = 262,144, d = 5,376 lay 9.3e-6 from the
+            // 64-bit ones; now 2.3e-6). An MFMA into tot itself chains the steps: 120.6 against
+            // 119.2 us.
             const bf16x8_t xa = __builtin_bit_cast(bf16x8_t, xRow[(U >> 1) * 4 * lrows]);
 #pragma unroll
             for (int j = 0; j < RT; ++j) {
                 const u32x4_t bp = u32x4_t{sq[s - 1][j].x, sq[s - 1][j].y, sq[s][j].x, sq[s][j].y};
-                bacc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, __builtin_bit_cast(bf16x8_t, bp),
-                                                                  bacc[j], 0, 0, 0);
+                const f32x4_t bias = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    xa, __builtin_bit_cast(bf16x8_t, bp), f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (i % MS == 0 || (NORM && i % MS == 1)) tot[j][0][i] += bias[i];
             }
             if constexpr (kReload) {
                 load_scales_ordered<RT>(rs, min(U - 1 + PF, last), vo_s, sq[s - 1]);
@@ -771,26 +842,37 @@ __global__ __launch_bounds__(NW * 64) void head_small_kernel(HeadArgs a) {
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto cycle = [&](uint32_t U0, auto reload) {
-        static_for<PF>([&](auto slot) { step(U0, slot, reload); });
-    };
-    for (uint32_t U0 = 0; U0 + PF < npad; U0 += PF) cycle(U0, std::true_type{});
-    cycle(npad - PF, std::false_type{});
-#pragma unroll
-    for (int j = 0; j < RT; ++j) tot[j][0] += bacc[j];
+    uint32_t U0 = 0;
+    for (; U0 + PF < npad; U0 += PF)
+        static_for<PF>([&](auto slot) { step(U0, slot, std::true_type{}); });
+    static_for<PF / 2>([&](auto pair) {
+        constexpr int s = 2 * decltype(pair)::value;
+        if (s == 0 || U0 + s < npad) {
+            step(U0, std::integral_constant<int, s>{}, std::false_type{});
+            step(U0, std::integral_constant<int, s + 1>{}, std::false_type{});
+        }
+    });
     if constexpr (NORM) {
-        // row lane / 16: the two halves' sums, times the row's 1 / sqrt(mean(x^2) + eps)
-        const uint32_t m = (lane >> 4) < a.M ? (lane >> 4) : 0u;
-        float t = 0.0f;
-        for (int w2 = 0; w2 < NW; ++w2) t += ss_red[w2][m];
-        const float rms = 1.0f / sqrtf(t / static_cast<float>(a.d) + a.eps);
+        // the two halves' sums, times the row's 1 / sqrt(mean(x^2) + eps)
 #pragma unroll
-        for (int j = 0; j < RT; ++j) tot[j][0][0] = (tot[j][0][0] + tot[j][0][1]) * rms;
+        for (int i = 0; i < 4; i += MS) {
+            // the row's partial square sums, over the 16 lanes that share it
+            const uint32_t r = (4 * (lane >> 4) + i) / MS, m = r < a.M ? r : 0u;
+            float t = 0.0f;
+            for (uint32_t u = lane & 15; u < npad / 2; u += 16) t += ss_red[m * (npad / 2) + u];
+            t += dpp_move<0xB1>(t, t);
+            t += dpp_move<0x4E>(t, t);
+            t += dpp_move<0x141>(t, t);
+            t += dpp_move<0x140>(t, t);
+            const float rms = 1.0f / sqrtf(t / static_cast<float>(a.d) + a.eps);
+#pragma unroll
+            for (int j = 0; j < RT; ++j) tot[j][0][i] = (tot[j][0][i] + tot[j][0][i + 1]) * rms;
+        }
     }
     if constexpr (MODE == kModeSample) {
-        head_epilogue_sample<RT, NW, MS>(a, tot, tile0, block_row0, cnt, exp2_tbl, prm);
+        head_epilogue_sample<RT, MS>(a, tot, tile0, block_row0, cnt, exp2_tbl, prm);
     } else {
-        head_epilogue<1, 4, RT, MODE, NW, MS>(a, tot, tile0, se);
+        head_epilogue<1, 4, RT, MODE, MS>(a, tot, tile0, se);
     }
 }
 
@@ -894,21 +976,19 @@ __global__ __launch_bounds__(kHeadThreads) void prep_rmsnorm_kernel(const float*
         const float xs[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
         const uint32_t ws[4] = {wv.x, wv.y, wv.z, wv.w};
         const float r = rms[row];
-        uint32_t half[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const uint32_t wb = (ws[e >> 1] >> (16 * (e & 1))) & 0xFFFFu;
-            const float he = (xs[e] * r) * __uint_as_float(wb << 16);  // x * rms * weight
-            const uint32_t hi = f32_to_bf16_rne(he);
-            const uint32_t lo = f32_to_bf16_rne(he - __uint_as_float(hi << 16));
-            half[e] = lo_plane ? lo : hi;
+        for (int e = 0; e < 4; ++e) {
+            const float h0 = (xs[2 * e] * r) * bf16_lo(ws[e]);  // x * rms * weight
+            const float h1 = (xs[2 * e + 1] * r) * bf16_hi(ws[e]);
+            const uint32_t hi = f32x2_to_bf16(h0, h1);
+            const uint32_t lo = f32x2_to_bf16(h0 - bf16_lo(hi), h1 - bf16_hi(hi));
+            v[e] = lo_plane ? lo : hi;
             // the group sum of what the MFMA rows carry, hi + lo (exact in fp32): the bias
             // term's X must cancel the MFMA's 128 X to the last bit, or the 2^-18 gap between
             // h and hi + lo comes back multiplied by 128 s
-            s += __uint_as_float(hi << 16) + __uint_as_float(lo << 16);
+            s += bf16_lo(hi) + bf16_lo(lo);
+            s += bf16_hi(hi) + bf16_hi(lo);
         }
-        v = u32x4_t{half[0] | (half[1] << 16), half[2] | (half[3] << 16), half[4] | (half[5] << 16),
-                    half[6] | (half[7] << 16)};
         if (lo_plane) s = 0.0f;  // the bias is added once, on the high rows
     }
     s += __shfl_xor(s, 1);
@@ -1192,7 +1272,7 @@ __device__ __forceinline__ void head_epilogue32(const HeadArgs& a, f32x16_t (&to
     const uint32_t j = lane & 31;
     const uint32_t m = 32 * (j / 16) + 8 * ((j % 16) >> 2) + mb + (j & 3);
     if (j < NM * 16 && m < TWD_MAX_ROWS) se.red[wave][m] = k[0];
-    grid_finish<NW>(a, se);
+    grid_finish(a, se);
 }
 
 // Block = NW waves; wave w owns NP tile pairs (32 vocabulary rows each, tiles T0 + 2 p and
@@ -1499,35 +1579,28 @@ struct twd_head {
     float softcap = 0.f;
     uint8_t* tiled = nullptr;
     uint64_t tiled_bytes = 0;
-    // [TWD_MAX_ROWS] per-row maxima (zero between launches), the arrival counter, and the
-    // repack's flag
+    // the finish state: the groups' per-row maxima (zero between launches) and the arrival
+    // counters (finish_max, kFinCtrWords), and the repack's flag
     uint64_t* gbest = nullptr;
     uint32_t epoch = kFirstEpoch - 1;  // of the last launch; the next is epoch_after(epoch)
+    uint32_t tree_epoch = kFirstEpoch - 1;  // of the last launch whose blocks finished in groups
     StreamOrder order;            // calls on several streams share gbest, hp/hx and sel
     u32x4_t* hp = nullptr;        // prepared h in A-fragment order for M > 8 (prep_hidden_kernel)
     u32x4_t* hx = nullptr;        // its bias A-fragment entries
     twd_selector* sel = nullptr;
     uint16_t* norm_w = nullptr;   // final RMSNorm weight, when loaded from a container
     SampleStats stats{};          // per-wave statistics of the fused sample pass (M <= 8)
-    uint32_t sample_blocks = 0;   // its head blocks for M <= 4 (0: no fused sample pass)
-    uint32_t sample_blocks8 = 0;  // for 5 <= M <= 8 (0: none, e.g. h and the counts exceed LDS)
+    uint32_t stats_cap = 0;       // its records per row (0: no fused sample pass)
 };
 
 namespace {
 
 // staged-h kernel (M <= 16): row tiles per wave, measured best on MI355X
 constexpr int kRT1 = 4;
-// resident-h kernel: row tiles per wave and weight units in flight, measured best on MI355X at
-// V = 262144, d = 5376: 4096 waves, 16 resident per CU, one round on 256 CUs. M <= 4: 512 blocks
-// of 8 waves, two per CU. 5 <= M <= 8: 256 blocks of 16 waves, one per CU (one LDS copy of h
-// serves 16 waves; M = 8 leaves no room for a second block's h anyway).
-constexpr int kRTS = 4, kPFS = 2;
-constexpr int kNWS4 = 8, kNWS8 = 16;
 constexpr size_t kLdsBytes = 160 * 1024;
-constexpr uint32_t kSmallMaxRows = 8;
-// static LDS of the 16-wave sample mode (its occurrence counts, 8 rows x 1,024 block rows, and
-// the exp table), beside the dynamic h staging
-constexpr size_t kSample8StaticLds = kSampleRows * kNWS8 * kRTS * kTileRows * 4 + 64 * 8 + 1024;
+constexpr uint32_t kCUs = 256;
+// upper bound of the resident-h kernel's static LDS (finish state, tables, square sums)
+constexpr size_t kResidentStaticLds = 4096;
 
 uint32_t blocks_for(uint32_t ntiles, int rt, int nw = kHeadWaves) {
     const uint32_t per = nw * rt;
@@ -1548,12 +1621,59 @@ int check_geometry(uint32_t vocab, uint32_t d, uint32_t group) {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Dynamic LDS of the resident-h kernel with ring depth PF: prepared h (M rows of npad chunks of
-// 256 B) + bias entries (npad / 2 super-units x 4 slices x M of 16 B).
-template <int PF>
-size_t small_smem_bytes(uint32_t rows, uint32_t d) {
-    const size_t npad = small_pad_units<PF>(d / kChunkK);
-    return static_cast<size_t>(rows) * npad * (256 + 32);
+// LDS of h staged by the resident-h kernel: per row, npad chunks of 256 B and npad / 2 bias
+// super-units of 4 slices of 16 B.
+size_t resident_h_bytes(uint32_t lds_rows, uint32_t nunits) {
+    return static_cast<size_t>(lds_rows) * resident_pad_units(nunits) * (256 + 32);
+}
+
+// How the resident-h kernel covers a head of `ntiles` row tiles: RT tiles per wave, nw waves per
+// block. RT is the smallest of 1, 2, 4 that leaves at most 16 waves per CU (four per SIMD, what
+// its registers allow), and the blocks are sized so that the waves spread evenly over all 256
+// CUs in one round: one block per CU up to 12 waves, two of half as many past that (a block's
+// staging and finish then overlap the other's stream) where two copies of h fit in LDS; with
+// more than four rows and exactly 16 waves, one block (half the staging). Larger heads take
+// further rounds of 8- or 16-wave blocks. Measured against four tiles per wave and 8- or
+// 16-wave blocks throughout (M = 1 / M = 5, greedy, us): V = 32,003 d = 2,048 (RT 1, 8 waves)
+// 19.2 -> 12.3 / 33.1 -> 13.7; V = 65,536 d = 4,096 (RT 1, 2 x 8 / 16) 36.6 -> 27.5 / 60.9 -> 29.7;
+// V = 100,003 d = 2,560 (RT 2, 2 x 7) 29.0 -> 27.1 / 42.7 -> 28.8; V = 151,669 d = 3,584 (RT 4,
+// 10) 64.3 -> 51.8 / 58.7 -> 53.8; V = 262,144 d = 5,376 unchanged. With the finish by groups and
+// h requested first, V = 32,003: 10.9 / 11.8; M = 12 26.7 -> 17.1.
+struct ResidentShape {
+    int ms = 0, rt = 0;        // rows MS apart in the MFMA's rows, RT tiles per wave
+    uint32_t nw = 0, blocks = 0;
+    size_t bytes = 0;          // dynamic LDS
+    bool tree = false;         // blocks count in by groups (grid_arrive_tree)
+    bool fits = false;
+};
+
+ResidentShape resident_shape(uint32_t ntiles, uint32_t nunits, uint32_t rows, bool norm, bool sample) {
+    ResidentShape s;
+    s.ms = rows <= 4 ? 4 : rows <= 8 ? 2 : 1;
+    s.rt = ntiles <= 16 * kCUs ? 1 : ntiles <= 32 * kCUs ? 2 : 4;
+    const size_t hb = resident_h_bytes(norm ? 2 * rows : rows, nunits);
+    auto bytes = [&](uint32_t nw) {  // the sample mode's occurrence counts lie past h
+        return hb + (sample ? static_cast<size_t>(16 / s.ms) * nw * s.rt * kTileRows * 4 : 0);
+    };
+    auto fit = [&](uint32_t nw, uint32_t copies) { return copies * (bytes(nw) + kResidentStaticLds) <= kLdsBytes; };
+    const uint32_t waves = (ntiles + s.rt - 1) / s.rt, per_cu = (waves + kCUs - 1) / kCUs;
+    if (per_cu > 16)
+        s.nw = s.ms == 4 && fit(8, 2) ? 8 : 16;
+    else if (per_cu > 12 && !(s.ms < 4 && per_cu == 16) && fit((per_cu + 1) / 2, 2))
+        s.nw = (per_cu + 1) / 2;
+    else
+        s.nw = std::max(per_cu, 4u);  // at least four waves to stage h
+    s.blocks = (waves + s.nw - 1) / s.nw;
+    s.bytes = bytes(s.nw);
+    // short streams, and more blocks than CUs, finish together
+    s.tree = s.rt == 1 || s.blocks > kCUs;
+    // Past eight rows the kernel is instantiated, and used, for one tile per wave only (at
+    // V = 100,003, d = 2,560 and above the staged-h kernel is as fast). Five to eight rows with
+    // the RMSNorm prologue take the staged-h kernel where it fills whole rounds too: 137.8 against
+    // 143.8 us at V = 262,144, d = 5,376, M = 5 (59.5 against 67.3 the other way at V = 151,669,
+    // d = 3,584; 68.2 against 73.2 at V = 240,003, d = 2,560).
+    s.fits = fit(s.nw, 1) && (s.ms > 1 || s.rt == 1) && !(norm && s.ms == 2 && s.rt == 4 && per_cu >= 16);
+    return s;
 }
 
 template <typename K>
@@ -1562,28 +1682,67 @@ hipError_t allow_smem(K kernel, size_t bytes) {
                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
 }
 
-// Lets every resident-h instantiation use the LDS it needs for kSmallMaxRows rows of d.
-int enable_small_kernels(uint32_t d) {
-    const size_t bytes4 = small_smem_bytes<kPFS>(4, d);
-    const size_t bytes8 = small_smem_bytes<kPFS>(kSmallMaxRows, d);
-    if (bytes4 + sizeof(EpiSharedT<kNWS4>) > kLdsBytes || bytes8 + sizeof(EpiSharedT<kNWS8>) > kLdsBytes)
-        return fail(TWD_E_UNSUPPORTED, "d_model too large for the LDS-resident head");
+// f(kernel) for the resident-h instantiation of a shape.
+template <int MODE, bool NORM, typename F>
+void with_resident(int ms, int rt, F&& f) {
+    auto by_rt = [&](auto msc) {
+        constexpr int MS = decltype(msc)::value;
+        if (rt == 1) {
+            f(head_small_kernel<MS, 1, 4, MODE, NORM>);
+        } else if constexpr (MS > 1) {
+            if (rt == 2)
+                f(head_small_kernel<MS, 2, 4, MODE, NORM>);
+            else
+                f(head_small_kernel<MS, 4, 2, MODE, NORM>);
+        }
+    };
+    if (ms == 4) return by_rt(std::integral_constant<int, 4>{});
+    if (NORM || MODE == kModeSample || ms == 2) return by_rt(std::integral_constant<int, 2>{});
+    if constexpr (!NORM && MODE != kModeSample) by_rt(std::integral_constant<int, 1>{});
+}
+
+// This launch's epochs; only greedy launches count in.
+template <int MODE>
+FinishEpochs finish_epochs(twd_head* h, bool tree) {
+    FinishEpochs ep{};
+    if (MODE != kModeGreedy) return ep;
+    h->epoch = epoch_after(h->epoch);
+    ep.epoch = h->epoch;
+    ep.next = epoch_after(h->epoch);
+    if (tree) {
+        h->tree_epoch = epoch_after(h->tree_epoch);
+        ep.tree_epoch = h->tree_epoch;
+        ep.tree_next = epoch_after(h->tree_epoch);
+    }
+    return ep;
+}
+
+template <int MODE, bool NORM>
+hipError_t launch_resident(const ResidentShape& s, const HeadArgs& a, hipStream_t stream) {
+    with_resident<MODE, NORM>(s.ms, s.rt, [&](auto kernel) {
+        kernel<<<s.blocks, s.nw * 64, s.bytes, stream>>>(a);
+    });
+    return hipGetLastError();
+}
+
+// Lets every resident-h instantiation use all of a CU's LDS.
+int enable_small_kernels(uint32_t nunits) {
+    if (nunits > kMaxUnits) return fail(TWD_E_UNSUPPORTED, "d_model too large for the LDS-resident head");
     hipError_t e = hipSuccess;
-    if (e == hipSuccess) e = allow_smem(head_small_kernel<4, kRTS, kPFS, kNWS4, kModeLogits>, bytes4);
-    if (e == hipSuccess) e = allow_smem(head_small_kernel<4, kRTS, kPFS, kNWS4, kModeGreedy>, bytes4);
-    if (e == hipSuccess) e = allow_smem(head_small_kernel<2, kRTS, kPFS, kNWS8, kModeLogits>, bytes8);
-    if (e == hipSuccess) e = allow_smem(head_small_kernel<2, kRTS, kPFS, kNWS8, kModeGreedy>, bytes8);
-    // the RMSNorm prologue variant: two LDS rows per h row, M <= 4
-    if (e == hipSuccess) e = allow_smem(head_small_kernel<4, kRTS, kPFS, kNWS4, kModeLogits, true>, bytes8);
-    if (e == hipSuccess) e = allow_smem(head_small_kernel<4, kRTS, kPFS, kNWS4, kModeGreedy, true>, bytes8);
-    if (e == hipSuccess) e = allow_smem(head_small_kernel<4, kRTS, kPFS, kNWS8, kModeLogits, true>, bytes8);
-    if (e == hipSuccess) e = allow_smem(head_small_kernel<4, kRTS, kPFS, kNWS8, kModeGreedy, true>, bytes8);
-    // the fused sample pass (M <= 4), with and without the RMSNorm prologue, and 5 <= M <= 8
-    // where its counts fit beside h
-    if (e == hipSuccess) e = allow_smem(head_small_kernel<4, kRTS, kPFS, kNWS4, kModeSample>, bytes4);
-    if (e == hipSuccess) e = allow_smem(head_small_kernel<4, kRTS, kPFS, kNWS4, kModeSample, true>, bytes8);
-    if (e == hipSuccess && bytes8 + kSample8StaticLds <= kLdsBytes)
-        e = allow_smem(head_small_kernel<2, kRTS, kPFS, kNWS8, kModeSample>, bytes8);
+    auto allow = [&](auto kernel) {
+        if (e == hipSuccess) e = allow_smem(kernel, kLdsBytes - kResidentStaticLds);
+    };
+    for (int rt = 1; rt <= 4; rt *= 2) {
+        for (int ms = 1; ms <= 4; ms *= 2) {
+            with_resident<kModeLogits, false>(ms, rt, allow);
+            with_resident<kModeGreedy, false>(ms, rt, allow);
+            if (ms == 1) continue;
+            with_resident<kModeLogits, true>(ms, rt, allow);
+            with_resident<kModeGreedy, true>(ms, rt, allow);
+            with_resident<kModeSample, false>(ms, rt, allow);
+            with_resident<kModeSample, true>(ms, rt, allow);
+        }
+    }
     if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
     return TWD_OK;
 }
@@ -1597,25 +1756,26 @@ int head_alloc(uint32_t vocab, uint32_t d, float softcap, twd_head** out) {
     h->nunits = d / kChunkK;
     h->tiled_bytes = static_cast<uint64_t>(h->ntiles) * h->nunits * kUnitBytes;
     hipError_t e = hipMalloc(&h->tiled, h->tiled_bytes);
-    // gbest: per-row maxima, the arrival counter's words, and the repack's bad-scale flag; the
-    // counter starts armed for the first launch's epoch
-    const uint64_t armed = kFirstEpoch;
-    constexpr size_t kWords = TWD_MAX_ROWS + kArriveWords + 1;
-    if (e == hipSuccess) e = hipMalloc(&h->gbest, sizeof(uint64_t) * kWords);
-    if (e == hipSuccess) e = hipMemset(h->gbest, 0, sizeof(uint64_t) * kWords);
-    if (e == hipSuccess) e = hipMemcpy(h->gbest + TWD_MAX_ROWS, &armed, sizeof(armed), hipMemcpyHostToDevice);
+    // gbest: maxima, the arrival counters' words, and the repack's bad-scale flag; the counters
+    // start armed for the first launch's epoch
+    std::vector<uint64_t> state(kFinishWords + 1, 0);
+    for (uint32_t g = 0; g <= kFinGroups; ++g) state[TWD_MAX_ROWS + kFinLine * g] = kFirstEpoch;
+    const size_t state_bytes = sizeof(uint64_t) * state.size();
+    if (e == hipSuccess) e = hipMalloc(&h->gbest, state_bytes);
+    if (e == hipSuccess) e = hipMemcpy(h->gbest, state.data(), state_bytes, hipMemcpyHostToDevice);
     // hp / hx: room past the last chunk and super-unit (each stage copies the next one
     // unconditionally)
     if (e == hipSuccess) e = hipMalloc(&h->hp, sizeof(u32x4_t) * (h->nunits + 3) * 4 * 4 * 64);
     if (e == hipSuccess) e = hipMalloc(&h->hx, sizeof(u32x4_t) * (super_units(h->nunits) + 1) * 4 * 64);
-    // the fused sample pass's wave records: rows <= 4 on 8-wave blocks, 5..8 on 16-wave blocks
-    // (the two grids' wave counts differ by less than a block); the 16-wave form also needs its
-    // occurrence counts beside h in LDS
-    const uint32_t sb = blocks_for(h->ntiles, kRTS, kNWS4), sb8 = blocks_for(h->ntiles, kRTS, kNWS8);
-    const uint32_t waves = std::max(sb * kNWS4, sb8 * kNWS8);
-    if (waves <= kSampleMaxWaves) {
-        h->sample_blocks = sb;
-        if (small_smem_bytes<kPFS>(kSampleRows, d) + kSample8StaticLds <= kLdsBytes) h->sample_blocks8 = sb8;
+    // the fused sample pass's wave records, for the shape with the most waves
+    uint32_t waves = 0;
+    for (uint32_t rows = 1; rows <= kSampleRows; ++rows)
+        for (int norm = 0; norm < 2; ++norm) {
+            const ResidentShape s = resident_shape(h->ntiles, h->nunits, rows, norm != 0, true);
+            if (s.fits && s.blocks * s.nw <= kSampleMaxWaves) waves = std::max(waves, s.blocks * s.nw);
+        }
+    h->stats_cap = waves;
+    if (waves != 0) {
         const size_t n = static_cast<size_t>(kSampleRows) * waves;
         if (e == hipSuccess) e = hipMalloc(&h->stats.key, n * sizeof(uint64_t));
         if (e == hipSuccess) e = hipMalloc(&h->stats.sum, n * sizeof(double));
@@ -1627,7 +1787,7 @@ int head_alloc(uint32_t vocab, uint32_t d, float softcap, twd_head** out) {
         twd_head_destroy(h);
         return hip_fail(e, "allocating the LM head");
     }
-    if (enable_small_kernels(d) != TWD_OK || twd_selector_create(vocab, TWD_MAX_ROWS, &h->sel) != TWD_OK) {
+    if (enable_small_kernels(h->nunits) != TWD_OK || twd_selector_create(vocab, TWD_MAX_ROWS, &h->sel) != TWD_OK) {
         twd_head_destroy(h);
         return TWD_E_HIP;
     }
@@ -1635,7 +1795,7 @@ int head_alloc(uint32_t vocab, uint32_t d, float softcap, twd_head** out) {
     return TWD_OK;
 }
 
-uint32_t* repack_flag(twd_head* h) { return reinterpret_cast<uint32_t*>(h->gbest + TWD_MAX_ROWS + kArriveWords); }
+uint32_t* repack_flag(twd_head* h) { return reinterpret_cast<uint32_t*>(h->gbest + kFinishWords); }
 
 int head_repack(twd_head* h, const uint8_t* wsb_dev, hipStream_t stream) {
     const uint64_t w_bytes = static_cast<uint64_t>(h->vocab) * (h->d / 8) * 4;
@@ -1670,19 +1830,15 @@ int launch_head(twd_head* h, const uint16_t* hidden, uint32_t rows, float* logit
     a.vocab = h->vocab;
     a.gbest = h->gbest;
     a.gctr = h->gbest + TWD_MAX_ROWS;
-    if (MODE != kModeLogits) h->epoch = epoch_after(h->epoch);  // only greedy launches count in
-    a.epoch = h->epoch;
-    a.next_epoch = epoch_after(h->epoch);
     a.tokens = tokens;
     a.drafts = drafts;
     a.n_drafts = n_drafts;
     a.vres = vres;
-    if (rows <= 4) {
-        head_small_kernel<4, kRTS, kPFS, kNWS4, MODE><<<blocks_for(h->ntiles, kRTS, kNWS4), kNWS4 * 64,
-                                                      small_smem_bytes<kPFS>(rows, h->d), stream>>>(a);
-    } else if (rows <= kSmallMaxRows) {
-        head_small_kernel<2, kRTS, kPFS, kNWS8, MODE><<<blocks_for(h->ntiles, kRTS, kNWS8), kNWS8 * 64,
-                                                      small_smem_bytes<kPFS>(rows, h->d), stream>>>(a);
+    const ResidentShape shape = resident_shape(h->ntiles, h->nunits, std::min(rows, 16u), false, false);
+    const bool resident = rows <= 16 && shape.fits;
+    a.ep = finish_epochs<MODE>(h, resident && shape.tree);
+    if (resident) {
+        TWD_HIP((launch_resident<MODE, false>(shape, a, stream)));
     } else if (rows <= 16) {
         prep_hidden_kernel<1><<<padded_units(h->nunits) * 1, kHeadThreads, 0, stream>>>(hidden, rows, h->d,
                                                                                        h->hp, h->hx);
@@ -1727,26 +1883,18 @@ int launch_head_rmsnorm(twd_head* h, const float* x, const uint16_t* norm_w, flo
     a.vocab = h->vocab;
     a.gbest = h->gbest;
     a.gctr = h->gbest + TWD_MAX_ROWS;
-    if (MODE != kModeLogits) h->epoch = epoch_after(h->epoch);  // only greedy launches count in
-    a.epoch = h->epoch;
-    a.next_epoch = epoch_after(h->epoch);
     a.tokens = tokens;
     a.drafts = drafts;
     a.n_drafts = n_drafts;
     a.vres = vres;
-    if (rows <= 4) {
+    const ResidentShape shape = resident_shape(h->ntiles, h->nunits, rows, true, false);
+    a.ep = finish_epochs<MODE>(h, shape.fits && shape.tree);
+    if (shape.fits) {
         // the resident-h kernel stages the normalised rows itself, two LDS rows each
         a.x = x;
         a.norm_w = norm_w;
         a.eps = eps;
-        const size_t bytes = small_smem_bytes<kPFS>(2 * rows, h->d);
-        if (2 * (bytes + sizeof(EpiSharedT<kNWS4>)) <= kLdsBytes)
-            head_small_kernel<4, kRTS, kPFS, kNWS4, MODE, true>
-                <<<blocks_for(h->ntiles, kRTS, kNWS4), kNWS4 * 64, bytes, stream>>>(a);
-        else
-            head_small_kernel<4, kRTS, kPFS, kNWS8, MODE, true>
-                <<<blocks_for(h->ntiles, kRTS, kNWS8), kNWS8 * 64, bytes, stream>>>(a);
-        TWD_HIP(hipGetLastError());
+        TWD_HIP((launch_resident<MODE, true>(shape, a, stream)));
         return TWD_OK;
     }
     a.fold = 1;
@@ -1759,14 +1907,15 @@ int launch_head_rmsnorm(twd_head* h, const float* x, const uint16_t* norm_w, flo
 
 // The fused sample pass: the resident-h kernel in sample mode (softcap, penalty from LDS
 // occurrence counts, logits store, per-wave statistics), then select_sample_merge_kernel. Used
-// for rows <= 8 (rows <= 4 with the RMSNorm prologue) when the head's wave count allows it, the
-// 16-wave form's counts fit beside h, and the rows' histories (where the penalty applies) hold
-// at most kSampleMaxHistory ids together: every head block scans them.
+// for rows <= 8 when the head's wave count allows it, h and the occurrence counts fit in LDS, and
+// the rows' histories (where the penalty applies) hold at most kSampleMaxHistory ids together:
+// every head block scans them.
 constexpr uint32_t kSampleMaxHistory = 16384;
 
 bool sample_fusable(const twd_head* h, uint32_t rows, const twd_row_params* params, bool norm) {
-    if (rows == 0 || rows > kSampleRows || h->sample_blocks == 0) return false;
-    if (rows > 4 && (norm || h->sample_blocks8 == 0)) return false;  // the RMSNorm form: rows <= 4
+    if (rows == 0 || rows > kSampleRows || h->stats_cap == 0) return false;
+    const ResidentShape s = resident_shape(h->ntiles, h->nunits, rows, norm, true);
+    if (!s.fits || s.blocks * s.nw > h->stats_cap) return false;
     uint64_t ids = 0;
     for (uint32_t m = 0; m < rows; ++m)
         if (params[m].repetition_penalty != 1.0f) ids += params[m].history_len;
@@ -1804,25 +1953,13 @@ int launch_head_sample(twd_head* h, const uint16_t* hidden, const float* x, cons
             return fail(TWD_E_INVALID, "null history with a non-empty history_len");
     }
     a.stats = h->stats;
-    uint32_t waves = 0;
-    if (x) {
-        const size_t bytes = small_smem_bytes<kPFS>(2 * rows, h->d);
-        head_small_kernel<4, kRTS, kPFS, kNWS4, kModeSample, true>
-            <<<h->sample_blocks, kNWS4 * 64, bytes, stream>>>(a);
-        waves = h->sample_blocks * kNWS4;
-    } else if (rows <= 4) {
-        head_small_kernel<4, kRTS, kPFS, kNWS4, kModeSample>
-            <<<h->sample_blocks, kNWS4 * 64, small_smem_bytes<kPFS>(rows, h->d), stream>>>(a);
-        waves = h->sample_blocks * kNWS4;
-    } else {  // rows two apart in the MFMA's rows, one 16-wave block per CU
-        head_small_kernel<2, kRTS, kPFS, kNWS8, kModeSample>
-            <<<h->sample_blocks8, kNWS8 * 64, small_smem_bytes<kPFS>(rows, h->d), stream>>>(a);
-        waves = h->sample_blocks8 * kNWS8;
-    }
-    TWD_HIP(hipGetLastError());
-    static_assert(kRTS * kTileRows == kSampleWaveRows, "a wave of the sample pass owns 64 rows");
-    return launch_sample_merge(h->stats, waves, logits, h->vocab, rows, params, tokens, h->sel->scratch.lng,
-                               stream);
+    const ResidentShape s = resident_shape(h->ntiles, h->nunits, rows, x != nullptr, true);
+    if (x)
+        TWD_HIP((launch_resident<kModeSample, true>(s, a, stream)));
+    else
+        TWD_HIP((launch_resident<kModeSample, false>(s, a, stream)));
+    return launch_sample_merge(h->stats, s.blocks * s.nw, static_cast<uint32_t>(s.rt) * kTileRows, logits, h->vocab,
+                               rows, params, tokens, h->sel->scratch.lng, stream);
 }
 
 // Runs one call's launches with the head's cross-stream ordering around them.

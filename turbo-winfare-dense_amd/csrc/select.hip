@@ -398,6 +398,7 @@ __global__ __launch_bounds__(kMergeThreads) void select_merge_kernel(SelectArgs 
 
 // ---- after the head's sample mode (or the wave-record pass): one block per row --------------------
 // sample_merge_row (select_core.h) finishes each row from its per-64-entry records.
+template <uint32_t RSH>
 __global__ __launch_bounds__(kSmThreads) void select_sample_merge_kernel(SelectArgs args_by_value,
                                                                          SampleMergeBufs b) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -409,7 +410,7 @@ __global__ __launch_bounds__(kSmThreads) void select_sample_merge_kernel(SelectA
     const SelectArgs& args = args_by_value;
 #endif
     const uint32_t row = blockIdx.x;
-    sample_merge_row(args.p[row], row, b, sh);
+    sample_merge_row<RSH>(args.p[row], row, b, sh);
 }
 
 // ---- shortlists longer than 256: top_k > 256 -------------------------------------------------------
@@ -450,6 +451,7 @@ struct LongBufs {
     uint64_t stride;
     uint32_t vocab;
     uint32_t waves;       // records per row
+    uint32_t rec_shift;   // log2 of the entries per record
     SampleStats st;       // [row][waves]
     uint64_t npad;        // sort buffer per long row: a power of two >= vocab
     uint64_t* keys;       // [n][npad]
@@ -537,7 +539,8 @@ __global__ __launch_bounds__(kLongThreads) void long_gather_kernel(LongArgs args
         }
     }
     __syncthreads();
-    const uint32_t nent = sh.c.misc[3] * kSampleWaveRows;
+    const uint32_t rsh = b.rec_shift, rmask = (1u << rsh) - 1u;
+    const uint32_t nent = sh.c.misc[3] << rsh;
     // the survivors into the sort buffer, eight loads requested at a time
     constexpr uint32_t kBatch = 8;
     const uint32_t per = (nent + NT - 1) / NT;
@@ -550,7 +553,7 @@ __global__ __launch_bounds__(kLongThreads) void long_gather_kernel(LongArgs args
             r[q] = 0xFFFFFFFFu;
             v[q] = 0.0f;
             if (i0 + q < per && f < nent) {
-                const uint32_t rr = sh.cwave[f / kSampleWaveRows] * kSampleWaveRows + f % kSampleWaveRows;
+                const uint32_t rr = (sh.cwave[f >> rsh] << rsh) + (f & rmask);
                 if (rr < b.vocab) {
                     r[q] = rr;
                     v[q] = lg[rr];
@@ -1085,8 +1088,8 @@ int long_reserve(LongScratch* l, uint32_t rows, uint64_t npad) {
 }
 }  // namespace
 
-int launch_long(LongScratch* lng, const SampleStats& st, uint32_t waves, const float* logits, uint64_t stride,
-                uint32_t vocab, uint32_t rows, const twd_row_params* params, uint32_t* tokens,
+int launch_long(LongScratch* lng, const SampleStats& st, uint32_t waves, uint32_t rec_rows, const float* logits,
+                uint64_t stride, uint32_t vocab, uint32_t rows, const twd_row_params* params, uint32_t* tokens,
                 hipStream_t stream) {
     LongArgs a{};
     for (uint32_t r = 0; r < rows; ++r) {
@@ -1107,6 +1110,7 @@ int launch_long(LongScratch* lng, const SampleStats& st, uint32_t waves, const f
     b.stride = stride;
     b.vocab = vocab;
     b.waves = waves;
+    b.rec_shift = static_cast<uint32_t>(__builtin_ctz(rec_rows));
     b.st = st;
     b.npad = npad;
     b.keys = lng->keys;
@@ -1149,10 +1153,12 @@ int enable_select_kernels() {
             err = hipFuncSetAttribute(reinterpret_cast<const void*>(select_merge_kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize,
                                       static_cast<int>(sizeof(MergeShared)));
-        if (err == hipSuccess)
-            err = hipFuncSetAttribute(reinterpret_cast<const void*>(select_sample_merge_kernel),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      static_cast<int>(sizeof(SampleMergeShared)));
+        for (const void* merge : {reinterpret_cast<const void*>(select_sample_merge_kernel<4>),
+                                  reinterpret_cast<const void*>(select_sample_merge_kernel<5>),
+                                  reinterpret_cast<const void*>(select_sample_merge_kernel<6>)})
+            if (err == hipSuccess)
+                err = hipFuncSetAttribute(merge, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          static_cast<int>(sizeof(SampleMergeShared)));
         if (err == hipSuccess)
             err = hipFuncSetAttribute(reinterpret_cast<const void*>(long_gather_kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1233,9 +1239,9 @@ int launch_select(const SelectScratch& s, float* logits, uint32_t vocab, uint32_
         mb.waves = waves;
         mb.st = st;
         mb.tokens = tokens;
-        select_sample_merge_kernel<<<rows, kSmThreads, sizeof(SampleMergeShared), stream>>>(a, mb);
+        select_sample_merge_kernel<kSampleWaveShift><<<rows, kSmThreads, sizeof(SampleMergeShared), stream>>>(a, mb);
         TWD_HIP(hipGetLastError());
-        return launch_long(s.lng, st, waves, logits, stride, vocab, rows, params, tokens, stream);
+        return launch_long(s.lng, st, waves, kSampleWaveRows, logits, stride, vocab, rows, params, tokens, stream);
     }
     SelectBufs b{};
     b.logits = logits;
@@ -1270,12 +1276,12 @@ int launch_select(const SelectScratch& s, float* logits, uint32_t vocab, uint32_
                          (reinterpret_cast<uintptr_t>(logits) & 15) == 0 && (stride & 3) == 0 ? 1u : 0u, st};
         wave_stats_kernel<1, false><<<dim3((vocab + kWsEntries - 1) / kWsEntries, rows), kWsThreads, 0, stream>>>(wb);
         TWD_HIP(hipGetLastError());
-        return launch_long(s.lng, st, waves, logits, stride, vocab, rows, params, tokens, stream);
+        return launch_long(s.lng, st, waves, kSampleWaveRows, logits, stride, vocab, rows, params, tokens, stream);
     }
     return TWD_OK;
 }
 
-int launch_sample_merge(const SampleStats& st, uint32_t waves, const float* logits, uint32_t vocab,
+int launch_sample_merge(const SampleStats& st, uint32_t waves, uint32_t rec_rows, const float* logits, uint32_t vocab,
                         uint32_t rows, const twd_row_params* params, uint32_t* tokens,
                         LongScratch* lng, hipStream_t stream) {
     if (waves == 0 || waves > kSampleMaxWaves) return fail(TWD_E_INVALID, "sample merge: head waves out of range");
@@ -1293,9 +1299,15 @@ int launch_sample_merge(const SampleStats& st, uint32_t waves, const float* logi
     b.waves = waves;
     b.st = st;
     b.tokens = tokens;
-    select_sample_merge_kernel<<<rows, kSmThreads, sizeof(SampleMergeShared), stream>>>(a, b);
+    auto merge = [&](auto kernel) { kernel<<<rows, kSmThreads, sizeof(SampleMergeShared), stream>>>(a, b); };
+    switch (rec_rows) {
+        case 16: merge(select_sample_merge_kernel<4>); break;
+        case 32: merge(select_sample_merge_kernel<5>); break;
+        case 64: merge(select_sample_merge_kernel<6>); break;
+        default: return fail(TWD_E_INVALID, "sample merge: record rows out of range");
+    }
     TWD_HIP(hipGetLastError());
-    return launch_long(lng, st, waves, logits, vocab, vocab, rows, params, tokens, stream);
+    return launch_long(lng, st, waves, rec_rows, logits, vocab, vocab, rows, params, tokens, stream);
 }
 
 int launch_verify_compare(const uint32_t* row_tokens, uint32_t rows, const uint32_t* drafts,

@@ -942,12 +942,14 @@ struct SampleMergeShared {
 // One row of the merge after the wave records (select_sample_merge_kernel's block, kSmThreads
 // threads): sample_token of row `row` with parameters p from its records and its penalised
 // logits (see the kernel's comment). Every thread of the block calls it.
-template <uint32_t PER>
+// RSH: log2 of the entries per record (4, 5 or 6).
+template <uint32_t PER, uint32_t RSH>
 __device__ __forceinline__ void sample_merge_row_per(const twd_row_params& p, uint32_t row, const SampleMergeBufs& b,
                                                      SampleMergeShared& sh) {
     constexpr int NT = kSmThreads;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t W = b.waves;
+    constexpr uint32_t rsh = RSH, rmask = (1u << rsh) - 1u;
     const size_t o = static_cast<size_t>(row) * W;
     const float* lg = b.logits + static_cast<size_t>(row) * b.stride;
 
@@ -1029,7 +1031,7 @@ __device__ __forceinline__ void sample_merge_row_per(const twd_row_params& p, ui
             one[q] = cand && !whole[q];
             wid[q] = w;
             wid1[q] = static_cast<uint16_t>(w);  // w < kSampleMaxWaves
-            bk[q] = rank_key(wm[q], w * kSampleWaveRows + (aux[q] & 63u));
+            bk[q] = rank_key(wm[q], (w << rsh) + (aux[q] & rmask));
             if (one[q] && __builtin_isfinite(wm[q])) smn = fminf(smn, wm[q]);
         }
         wave_put_n(whole, wid, &sh.c.misc[3], sh.cwave, kSmMaxCand);
@@ -1045,13 +1047,13 @@ __device__ __forceinline__ void sample_merge_row_per(const twd_row_params& p, ui
     if (all_waves) smn = INFINITY;
     // the gathered survivors follow the best ranks already listed (counted in misc[4] from 0)
     const uint32_t first = all_waves ? 0u : ncw1;
-    const uint32_t nent = all_waves ? W * kSampleWaveRows : ncw * kSampleWaveRows;  // entries to scan
+    const uint32_t nent = (all_waves ? W : ncw) << rsh;  // entries to scan
     // every candidate wave's entries, for the overflow path: the whole ones, then the others
-    const uint32_t nent_all = all_waves ? nent : (ncw + ncw1) * kSampleWaveRows;
+    const uint32_t nent_all = all_waves ? nent : (ncw + ncw1) << rsh;
     auto entry_row = [&](uint32_t f) -> uint32_t {
-        const uint32_t s = f / kSampleWaveRows;
+        const uint32_t s = f >> rsh;
         const uint32_t w = all_waves ? s : (s < ncw ? sh.cwave[s] : static_cast<uint32_t>(sh.cwave1[s - ncw]));
-        return w * kSampleWaveRows + f % kSampleWaveRows;
+        return (w << rsh) + (f & rmask);
     };
 
     // ---- survivors: entries in bins <= b* of the waves read whole, kGatherBatch loads at a time
@@ -1066,13 +1068,13 @@ __device__ __forceinline__ void sample_merge_row_per(const twd_row_params& p, ui
 #pragma unroll
         for (uint32_t q = 0; q < kGatherBatch; ++q) {
             const uint32_t f = (i0 + q) * NT + static_cast<uint32_t>(tid);
-            const uint32_t slot = min(f / kSampleWaveRows, kSmMaxCand - 1);
-            w[q] = all_waves ? f / kSampleWaveRows : sh.cwave[slot];
+            const uint32_t slot = min(f >> rsh, kSmMaxCand - 1);
+            w[q] = all_waves ? f >> rsh : sh.cwave[slot];
         }
 #pragma unroll
         for (uint32_t q = 0; q < kGatherBatch; ++q) {
             const uint32_t f = (i0 + q) * NT + static_cast<uint32_t>(tid);
-            const uint32_t rr = w[q] * kSampleWaveRows + f % kSampleWaveRows;
+            const uint32_t rr = (w[q] << rsh) + (f & rmask);
             const bool ok = i0 + q < per && f < nent && rr < b.vocab;
             r[q] = ok ? rr : 0xFFFFFFFFu;
             v[q] = lg[ok ? rr : 0u];
@@ -1239,12 +1241,13 @@ __device__ __forceinline__ void sample_merge_row_per(const twd_row_params& p, ui
 
 // One row of the merge: the records per thread sized to the row's record count, so that rows of
 // at most 4,096 records (V <= 262,144) run no code for records that do not exist.
+template <uint32_t RSH>
 __device__ __forceinline__ void sample_merge_row(const twd_row_params& p, uint32_t row, const SampleMergeBufs& b,
                                                  SampleMergeShared& sh) {
     if (b.waves <= kSmThreads * (kSmPer / 2))
-        sample_merge_row_per<kSmPer / 2>(p, row, b, sh);
+        sample_merge_row_per<kSmPer / 2, RSH>(p, row, b, sh);
     else
-        sample_merge_row_per<kSmPer>(p, row, b, sh);
+        sample_merge_row_per<kSmPer, RSH>(p, row, b, sh);
 }
 
 // ---- the wave records of logits in memory ------------------------------------------------------------

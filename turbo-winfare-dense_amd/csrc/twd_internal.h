@@ -113,7 +113,8 @@ __device__ __forceinline__ void top2_step(uint64_t& b1, uint64_t& b2) {
     top2_merge(b1, b2, o1, o2);
 }
 
-// A record's second word: the best rank's row within the record's 64 (bits 0-5), and the
+// A record's second word: the best rank's row modulo 64 (bits 0-5: a record holds 16, 32 or 64
+// consecutive rows from a multiple of their number), and the
 // second-best rank's value rounded up to bf16 (bits 16-31; -inf when there is none). Rounding up
 // keeps the merge's test conservative: a second value whose bin lies past b* rounds to one that
 // does too only when the exact one does.
@@ -339,6 +340,44 @@ __device__ __forceinline__ bool grid_arrive(unsigned long long* ctr, uint32_t nb
     return last;
 }
 
+// Arrivals in two levels. Atomics on one address are served one after another (about 11 ns each
+// on MI355X: 512 blocks that finish together spend 5 us on one counter, and as long again on one
+// maximum), so a launch's blocks count in on kFinGroups counters first, block b on counter
+// b % kFinGroups, each on a 128-byte line of its own, and the last block of each group counts in
+// on the launch's counter: 512 blocks then wait for 32 + 16 atomics in a row. The second level is
+// one more round trip, so launches whose blocks finish far apart anyway count in on the launch's
+// counter alone (tree_epoch 0). Every counter is grid_arrive's, the groups' with epochs of their
+// own (their launches are not every launch); exactly one block returns true, after every other
+// block of the launch counted in.
+// ctr: the launch's counter, then (from kFinLine words on) the groups', kFinLine words apart.
+constexpr uint32_t kFinGroups = 16;
+constexpr uint32_t kFinLine = 16;  // 64-bit words in 128 bytes
+constexpr uint32_t kFinCtrWords = kFinLine * (1 + kFinGroups);
+static_assert(kArriveWords <= kFinLine, "a counter fits its line");
+
+// epoch, next: of every launch; tree_epoch, tree_next: of the launches that use the groups (0: not
+// this one).
+struct FinishEpochs {
+    uint32_t epoch, next, tree_epoch, tree_next;
+};
+
+// The group of a block (0 without groups).
+__device__ __forceinline__ uint32_t finish_group(const FinishEpochs& ep, uint32_t block) {
+    return ep.tree_epoch != 0 ? block % kFinGroups : 0u;
+}
+
+__device__ __forceinline__ bool grid_arrive_tree(unsigned long long* ctr, uint32_t block, uint32_t nb,
+                                                 const FinishEpochs& ep) {
+    uint32_t top = nb;
+    if (ep.tree_epoch != 0) {
+        const uint32_t g = finish_group(ep, block);
+        const uint32_t size = nb / kFinGroups + (g < nb % kFinGroups ? 1u : 0u);
+        if (!grid_arrive(ctr + kFinLine * (1 + g), size, ep.tree_epoch, ep.tree_next)) return false;
+        top = nb < kFinGroups ? nb : kFinGroups;
+    }
+    return grid_arrive(ctr, top, ep.epoch, ep.next);
+}
+
 // bf16 bit patterns <-> float
 __device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
@@ -373,7 +412,8 @@ void order_release(StreamOrder& o);
 
 // ---- the fused sample pass ------------------------------------------------------------------------
 // The resident-h head kernel's sample mode publishes, per row m and wave w of the grid (index
-// m * waves + w), the selection statistics of the wave's 64 vocabulary rows [64 w, 64 w + 64);
+// m * waves + w), the selection statistics of the wave's R = 16, 32 or 64 vocabulary rows
+// [R w, R w + R);
 // select_sample_merge_kernel finishes the rows from them and the penalised logits.
 struct SampleStats {
     uint64_t* key;  // best rank (value desc, index asc) of the wave's rows (0: none live)
@@ -405,7 +445,8 @@ __host__ __device__ inline float fixed_ref(float cap, const twd_row_params& p) {
     return c <= kFixedRefMaxCap ? c : __builtin_nanf("");
 }
 constexpr uint32_t kSampleMaxWaves = 8192;  // waves a fused sample pass may have
-constexpr uint32_t kSampleWaveRows = 64;    // vocabulary rows per wave
+constexpr uint32_t kSampleWaveRows = 64;    // entries per record of the wave-record pass
+constexpr uint32_t kSampleWaveShift = 6;    // its log2
 
 // Sort and finish buffers of the rows whose shortlist is longer than kMaxWant (top_k > 256),
 // grown on demand by the calls that have such rows.
@@ -426,15 +467,17 @@ inline bool long_row(const twd_row_params& p, uint32_t vocab) {
 }
 
 // Enqueues the long path for those of `rows` rows that need it, after their penalised logits
-// and wave records (`waves` per row, row stride of the records) are in place. `lng` may be
+// and wave records (`waves` per row, row stride of the records, of rec_rows entries each) are in
+// place. `lng` may be
 // null only when no row needs it.
-int launch_long(LongScratch* lng, const SampleStats& st, uint32_t waves, const float* logits, uint64_t stride,
+int launch_long(LongScratch* lng, const SampleStats& st, uint32_t waves, uint32_t rec_rows, const float* logits,
+                uint64_t stride,
                 uint32_t vocab, uint32_t rows, const twd_row_params* params, uint32_t* tokens,
                 hipStream_t stream);
 
 // Enqueues the merge after a sample-mode head pass over `rows` rows (params: host array), and
 // the long path for rows with top_k > 256 (lng: their scratch).
-int launch_sample_merge(const SampleStats& st, uint32_t waves, const float* logits, uint32_t vocab,
+int launch_sample_merge(const SampleStats& st, uint32_t waves, uint32_t rec_rows, const float* logits, uint32_t vocab,
                         uint32_t rows, const twd_row_params* params, uint32_t* tokens,
                         LongScratch* lng, hipStream_t stream);
 

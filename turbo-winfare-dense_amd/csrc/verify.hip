@@ -1260,7 +1260,7 @@ __global__ __launch_bounds__(kRejThreads) void seg_sum_kernel(DraftArgs a, const
         const uint32_t row = r - 2 * a.npos;
         twd_row_params p = sel.base;
         p.uniform = sel.u[row];
-        sample_merge_row(p, row, sel.mb, u.sm);
+        sample_merge_row<kSampleWaveShift>(p, row, sel.mb, u.sm);
         return;
     }
     SeqShared& sh = u.seg.sh;
