@@ -1,0 +1,106 @@
+"""Shortlists of 257 to 4,096 entries, finished by one block per row: every way it can go -- records
+that bound the shortlist, records too few to (every entry a candidate), the gather overfull, its last
+fine bin overfull too (ties), a bin too full to rank by counting, dead entries, prefixes exactly on a
+threshold, and the lengths on both sides of its limit. Ids are compared with the oracle's sample_token
+on the same row, exactly."""
+import numpy as np
+import pytest
+
+from helpers import twd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def env():
+    import torch
+    t = twd()
+    sel = t.Selector(262144, 16)
+    yield torch, torch.device("cuda:0"), t, sel
+    sel.close()
+
+
+def row_of(kind, n, seed):
+    rng = np.random.default_rng(seed)
+    z = (3.6 * rng.standard_normal(n)).astype(np.float32)
+    if kind == "ties":          # some 40 distinct values
+        return (np.round(z * 2) / 2).astype(np.float32)
+    if kind == "equal":
+        return np.full(n, 1.25, np.float32)
+    if kind == "steps":         # three values: the last fine bin holds a third of the row
+        return rng.integers(0, 3, n).astype(np.float32)
+    if kind == "masked":        # 300 live entries, the rest one large negative number
+        out = np.full(n, -1e9, np.float32)
+        at = rng.choice(n, min(n, 300), replace=False)
+        out[at] = z[at]
+        return out
+    if kind == "minus_inf":     # 120 live entries, the rest -inf
+        out = np.full(n, -np.inf, np.float32)
+        at = rng.choice(n, min(n, 120), replace=False)
+        out[at] = z[at]
+        return out
+    if kind == "close":         # a span of a few ulps
+        return (np.float32(20.0) + rng.integers(0, 4000, n).astype(np.float32) * np.float32(2e-6)).astype(np.float32)
+    if kind == "outlier":       # one value far above: the others share few bins
+        z[n // 3] = 500.0
+        return z
+    return z
+
+
+KINDS = ["normal", "ties", "equal", "steps", "masked", "minus_inf", "close", "outlier"]
+
+
+def check(env, oracle, rows, params, V):
+    torch, dev, t, sel = env
+    lg = torch.from_numpy(np.stack(rows)).to(dev)
+    got = sel.select(lg, params).cpu().numpy().astype(np.int64) & 0xFFFFFFFF
+    for i, p in enumerate(params):
+        want = oracle.sample_token(rows[i], p.temperature, p.top_p, p.top_k, u=p.uniform)
+        assert int(got[i]) == want, (V, i, p.top_k, p.top_p, p.temperature)
+
+
+@pytest.mark.ties
+@pytest.mark.parametrize("V", [300, 4097, 8193, 32003, 262144])
+@pytest.mark.parametrize("k", [257, 1000, 4095, 4096, 4097])
+def test_kinds_of_rows(env, oracle, V, k):
+    t = env[2]
+    rng = np.random.default_rng(V + k)
+    rows, params = [], []
+    for i, kind in enumerate(KINDS):
+        for p in (0.93, 1.0):
+            rows.append(row_of(kind, V, 100 * i + k))
+            params.append(t.RowParams(float(rng.choice([0.5, 0.9, 1.7])), p, k, 1.0,
+                                      float(np.float32(rng.uniform(0, 0.9999))), 0.0, 0, 0))
+    check(env, oracle, rows, params, V)
+
+
+@pytest.mark.ties
+def test_prefixes_on_the_thresholds(env, oracle):
+    # equal entries: every weight is 1, so u = j / 2048 puts r exactly on a running sum, and
+    # p = i / 4096 of V = 4,096 equal entries puts p on (or an ulp from) a top-p prefix
+    t = env[2]
+    V = 4096
+    rows, params = [], []
+    for j in (1, 2, 700, 2047):
+        rows.append(row_of("equal", V, 0))
+        params.append(t.RowParams(0.7, 1.0, 2048, 1.0, j / 2048, 0.0, 0, 0))
+    for i in (1, 3, 512, 1365, 2048):
+        rows.append(row_of("equal", V, 0))
+        params.append(t.RowParams(0.7, i / 4096, 3000, 1.0, 0.999, 0.0, 0, 0))
+    check(env, oracle, rows, params, V)
+
+
+def test_odd_temperatures_and_draws(env, oracle):
+    # NaN and infinite temperatures (weights NaN or 1), u = 0, and rows with a NaN
+    torch, dev, t, sel = env
+    V = 32003
+    rows = [row_of("normal", V, 1), row_of("normal", V, 2), row_of("minus_inf", V, 3), row_of("normal", V, 4)]
+    params = [t.RowParams(float("nan"), 0.95, 700, 1.0, 0.3, 0.0, 0, 0),
+              t.RowParams(float("inf"), 0.99, 700, 1.0, 0.6, 0.0, 0, 0),
+              t.RowParams(float("inf"), 1.0, 700, 1.0, 0.6, 0.0, 0, 0),
+              t.RowParams(1.0, 0.9, 700, 1.0, 0.0, 0.0, 0, 0)]
+    check(env, oracle, rows, params, V)
+    bad = row_of("normal", V, 5)
+    bad[7] = np.nan
+    tok = sel.select(torch.from_numpy(bad[None]).to(dev), [t.RowParams(1.0, 0.9, 700, 1.0, 0.5, 0.0, 0, 0)])
+    assert int(tok.item()) & 0xFFFFFFFF == t.TOKEN_DEGENERATE

@@ -417,8 +417,9 @@ __global__ __launch_bounds__(kSmThreads) void select_sample_merge_kernel(SelectA
 //
 // sample_token takes any top_k: its shortlist is the top want = min(top_k, V) entries in the
 // order (value desc, index asc), and steps 5-7 run over all of them (sampling.cpp:120-168).
-// Rows with temperature > 0 and want > 256 are finished here, from the penalised logits and the
-// same wave records as the shorter rows (so the same row max and total):
+// Rows with temperature > 0 and want > 256 are finished from the penalised logits and the same
+// wave records as the shorter rows (so the same row max and total): those of up to kWideMax entries
+// by the wide kernels below, longer ones by these:
 //   * long_gather_kernel, one block per row: records_stats, then every entry of a candidate wave
 //     (maximum in a bin <= b*) that lies in a bin <= b*, into the row's sort buffer in any
 //     order. Every top-`want` entry is among them. The buffer is padded with zero ranks (below
@@ -459,6 +460,7 @@ struct LongBufs {
     uint32_t* len;        // [n] sort length (0: the row is already finished)
     float* gmax;          // [n]
     double* total;        // [n]
+    struct WideState* wide;  // [n] rows of up to kWideMax entries
     uint32_t* tokens;
 };
 
@@ -655,20 +657,18 @@ struct LongFinishShared {
     uint32_t best;
 };
 
-__global__ __launch_bounds__(kLongThreads) void long_finish_kernel(LongArgs args_by_value, LongBufs b) {
+// Steps 5-7 of long row j over its sorted ranks in b.keys. One block of kLongThreads threads; every
+// thread calls.
+__device__ __noinline__ void long_finish_row(const LongArgs& args, const LongBufs& b, uint32_t j, float gmax,
+                                             double total, LongFinishShared& sh) {
     constexpr int NT = kLongThreads;
-    __shared__ LongFinishShared sh;
-    const LongArgs& args = TWD_LONG_ARGS(args_by_value);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t j = blockIdx.x;
-    if (b.len[j] == 0) return;  // degenerate: long_gather_kernel wrote its token
     const uint32_t row = args.row[j];
     const twd_row_params p = args.p[j];
     const uint64_t* keys = b.keys + static_cast<size_t>(j) * b.npad;
     double* pre = b.pre + static_cast<size_t>(j) * b.npad;
     const uint32_t want = min(static_cast<uint32_t>(p.top_k), b.vocab);
-    const double mx = static_cast<double>(b.gmax[j]);
-    double total = b.total[j];
+    const double mx = static_cast<double>(gmax);
     const double td = static_cast<double>(p.temperature);
     const bool topp = p.top_p < 1.0f;
     const double pp = static_cast<double>(p.top_p);
@@ -751,7 +751,7 @@ __global__ __launch_bounds__(kLongThreads) void long_finish_kernel(LongArgs args
         if (sh.misc[2] == 0) break;
         if (wave == 0) {
             const double t = exact_row_total(RowSrc{b.logits + static_cast<size_t>(row) * b.stride, b.vocab,
-                                                    b.gmax[j], 0u}, sh.e);
+                                                    gmax, 0u}, sh.e);
             if (lane == 0) sh.total = t;
         }
         __syncthreads();
@@ -774,6 +774,521 @@ __global__ __launch_bounds__(kLongThreads) void long_finish_kernel(LongArgs args
         if (pre[i] >= r) atomicMin(&sh.best, i);
     __syncthreads();
     if (tid == 0) b.tokens[row] = rank_index(keys[sh.best]);
+}
+
+__global__ __launch_bounds__(kLongThreads) void long_finish_kernel(LongArgs args_by_value, LongBufs b) {
+    __shared__ LongFinishShared sh;
+    const LongArgs& args = TWD_LONG_ARGS(args_by_value);
+    const uint32_t j = blockIdx.x;
+    if (b.len[j] == 0) return;  // degenerate: long_gather_kernel wrote its token
+    long_finish_row(args, b, j, b.gmax[j], b.total[j], sh);
+}
+
+// ---- shortlists of 257 to kWideMax entries ---------------------------------------------------------
+//
+// The long path above moves every candidate through memory and sorts it over as many launches as the
+// longest possible buffer needs: 25 launches and 150 us for eight rows of V = 262,144 at
+// top_k = 1,000, most of them sort stages that no row reached. A shortlist of up to kWideMax
+// entries fits a CU's LDS, with room for the entries that share its last bin:
+//   * wide_filter_kernel<false>, `parts` blocks per row: the row's statistics and b* from its
+//     records, as the merge takes them, then the entries in bins <= b* of the block's share of the
+//     candidate records (every parts-th one), appended to the row's list in memory. One block per
+//     row is not enough for this: some 50 instructions per entry, 25 us for 65,000 entries on one CU;
+//   * where the records are too few to bound the shortlist (want near or past their number: every
+//     entry would be a candidate), wide_filter_kernel<true> first counts the entries in kFineBins
+//     bins of distance from the row max, and the list takes the fine bins up to the one that holds
+//     the want-th entry;
+//   * wide_finish_kernel, one block per row, all in LDS: a bucket sort (an entry's place is its fine
+//     bin's start plus the entries of the bin above it; a bitonic sort when a bin holds more than
+//     kWideBucket), then steps 5-7 by prefix sums over the block with finish_sums_par's margins. Its
+//     bound holds here: a running sum of up to 4,096 terms lies within 4,096 x 2^-53 of the exact
+//     one, so the parallel prefixes and the reference's differ by less than 2^-40, against the
+//     margin of 2^-36. A decision within the margin takes long_finish_row's sums, the reference's
+//     own. A list longer than kWideCap (ties) is gathered again by this block, by fine bins and, if
+//     the last bin alone is too long, above the want-th rank that a radix select finds.
+// Entries that dead_distance marks can be neither cut nor drawn and are left out, as in the merge.
+// Eight rows of V = 262,144 at top_k = 1,000: 150 -> 28.4 us.
+constexpr uint32_t kWideMax = 4096;    // longest shortlist
+constexpr uint32_t kWideCap = 8192;    // longest list
+constexpr uint32_t kFineBins = 2048;
+constexpr uint32_t kWideBucket = 192;  // entries of one fine bin ranked against each other
+constexpr uint32_t kPartCap = 4096;    // list entries of one filter block
+
+// The records bound the shortlist: with want below three quarters of their number, the entries above
+// the want-th maximum are some 1.4 times as many (64 entries per record, in any order).
+__device__ __host__ inline bool wide_needs_bins(uint32_t want, uint32_t waves) {
+    return 4u * want > 3u * (waves < 4096u ? waves : 4096u);
+}
+
+// A draw outside [0, 1) can fall past every weight, on the last survivor, dead or not.
+__device__ __forceinline__ double wide_dead(const twd_row_params& p) {
+    return p.uniform >= 0.0f && p.uniform < 1.0f ? dead_distance(p) : -INFINITY;
+}
+
+struct FineBin {
+    float gm, scale;
+    __device__ __forceinline__ uint32_t operator()(float x) const {
+        const float dist = (gm - x) * scale;  // scale 0: no bins
+        return dist < static_cast<float>(kFineBins - 1) ? static_cast<uint32_t>(dist) : kFineBins - 1;
+    }
+};
+
+// The records' bins in eight parts each; over twice their range where the shortlist can reach below
+// the smallest record maximum, which is where that range ends.
+__device__ __forceinline__ FineBin fine_bins(float gm, float scale, bool beyond) {
+    return FineBin{gm, scale * (static_cast<float>(kFineBins) / kBins) * (beyond ? 0.5f : 1.0f)};
+}
+
+// hist[0..kFineBins) to its inclusive prefix sums: two bins per thread.
+__device__ __forceinline__ void fine_scan(uint32_t* hist, uint32_t* wsum) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    static_assert(kFineBins == 2 * kLongThreads, "two bins per thread");
+    const uint32_t a = hist[2 * tid], b = hist[2 * tid + 1];
+    uint32_t x = wave_incl_scan_u32(a + b);
+    if (lane == 63) wsum[wave] = x;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) x += wsum[w];
+    hist[2 * tid] = x - b;
+    hist[2 * tid + 1] = x;
+    __syncthreads();
+}
+
+// The first fine bin by which `want` entries have been counted (the last one when fewer are there):
+// hist holds inclusive sums. Every thread calls; *out is shared.
+__device__ __forceinline__ uint32_t fine_bound(const uint32_t* hist, uint32_t want, uint32_t* out) {
+    if (threadIdx.x == 0) *out = kFineBins - 1;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < kFineBins; i += blockDim.x)
+        if (hist[i] >= want && (i == 0 || hist[i - 1] < want)) *out = i;  // one writer at most
+    __syncthreads();
+    return *out;
+}
+
+// f(value, row, in range) over the entries of the records listed in cwave[0..ncw), kBatch loads per
+// thread requested together; the same trip count in every thread.
+template <typename F>
+__device__ __forceinline__ void for_entries(const uint16_t* cwave, uint32_t ncw, uint32_t rsh, uint32_t vocab,
+                                            const float* lg, F&& f) {
+    constexpr int NT = kLongThreads;
+    constexpr uint32_t kBatch = 8;
+    const uint32_t rmask = (1u << rsh) - 1u, nent = ncw << rsh, per = (nent + NT - 1) / NT;
+    for (uint32_t i0 = 0; i0 < per; i0 += kBatch) {
+        float v[kBatch];
+        uint32_t r[kBatch];
+        bool in[kBatch];
+#pragma unroll
+        for (uint32_t q = 0; q < kBatch; ++q) {
+            const uint32_t e = (i0 + q) * NT + threadIdx.x;
+            r[q] = e < nent ? (static_cast<uint32_t>(cwave[e >> rsh]) << rsh) + (e & rmask) : 0xFFFFFFFFu;
+            in[q] = r[q] < vocab;
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < kBatch; ++q) v[q] = lg[in[q] ? r[q] : 0u];
+        f(v, r, in);
+    }
+}
+
+// A row's statistics from the filter's first block for the finish, its list's length and its fine
+// counts. n and hist are zero between calls: the finish clears them.
+struct WideState {
+    double total;
+    float gm, scale;
+    uint32_t bstar, degenerate;
+    uint32_t n;
+    uint32_t hist[kFineBins];
+};
+
+struct WideFilterShared {
+    uint64_t keys[kPartCap];
+    uint16_t cwave[kSampleMaxWaves];
+    uint32_t hist[kFineBins];
+    uint32_t wsum[16], base, bound;
+    TopScratch t;
+    SelCommon c;
+};
+
+template <bool COUNT>
+__global__ __launch_bounds__(kLongThreads) void wide_filter_kernel(LongArgs args_by_value, LongBufs b) {
+    constexpr int NT = kLongThreads;
+    static_assert(NT == kSmThreads, "records_stats' block");
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    WideFilterShared& sh = *reinterpret_cast<WideFilterShared*>(smem_raw);
+    const LongArgs& args = TWD_LONG_ARGS(args_by_value);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t part = blockIdx.x, parts = gridDim.x, j = blockIdx.y;
+    const uint32_t row = args.row[j];
+    const twd_row_params p = args.p[j];
+    const uint32_t W = b.waves;
+    const size_t o = static_cast<size_t>(row) * W;
+    const float* lg = b.logits + static_cast<size_t>(row) * b.stride;
+    WideState& st = b.wide[j];
+    const uint32_t want = min(static_cast<uint32_t>(p.top_k), b.vocab);  // <= kWideMax
+    const bool binned = wide_needs_bins(want, W);
+    if (COUNT && !binned) return;
+    const double dead = wide_dead(p);
+
+    float wm[kSmPer];
+    bool live[kSmPer];
+    uint32_t nan = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < kSmPer; ++q) {
+        const uint32_t i = tid + NT * q;
+        live[q] = i < W;
+        wm[q] = live[q] ? b.st.max[o + i] : -INFINITY;
+        nan |= wm[q] != wm[q] ? 1u : 0u;
+    }
+    float gm, scale;
+    uint32_t bstar = 0;
+    if (COUNT || !binned) {
+        // the statistics; the first block also the row total
+        double wsum[kSmPer];
+        if (tid < 64) sh.c.exp2_tbl[tid] = kExp2Table[tid];
+        if (part == 0) {
+#pragma unroll
+            for (uint32_t q = 0; q < kSmPer; ++q) wsum[q] = live[q] ? b.st.sum[o + tid + NT * q] : 0.0;
+        }
+        for (uint32_t i = tid; i < kReps * kBins; i += NT) sh.t.hist[i] = 0;
+        if constexpr (COUNT)
+            for (uint32_t i = tid; i < kFineBins; i += NT) sh.hist[i] = 0;
+        const float ref = fixed_ref(b.st.cap, p);
+        const RecStats rs = records_stats<false, kSmPer>(live, wm, nan, wsum, ref, want, sh.t, sh.c, dead);
+        bool degenerate = rs.degenerate;
+        double total = 0.0;
+        if (part == 0 && !degenerate) {
+            const double share = records_part<kSmPer>(wsum, wm, rs.gm, ref, sh.c.exp2_tbl);
+            if (lane == 0) sh.c.redd[wave] = share;
+            __syncthreads();
+            for (int w = 0; w < NT / 64; ++w) total += sh.c.redd[w];
+            degenerate = !(total > 0.0);  // sampling.cpp:116-118
+        }
+        if (part == 0 && tid == 0) {
+            st.total = total;
+            st.gm = rs.gm;
+            st.scale = rs.scale;
+            st.bstar = rs.bstar;
+            st.degenerate = degenerate ? 1u : 0u;
+        }
+        if (degenerate) return;
+        gm = rs.gm;
+        scale = rs.scale;
+        bstar = rs.bstar;
+    } else {  // after the counting launch
+        if (st.degenerate != 0) return;
+        gm = st.gm;
+        scale = st.scale;
+        for (uint32_t i = tid; i < kFineBins; i += NT) sh.hist[i] = st.hist[i];
+        if (tid == 0) sh.c.misc[3] = sh.c.misc[4] = 0;
+        __syncthreads();
+        fine_scan(sh.hist, sh.wsum);
+        bstar = fine_bound(sh.hist, want, &sh.bound);
+    }
+    const double dgm = static_cast<double>(gm);
+    RecStats coarse{};
+    coarse.gm = gm;
+    coarse.scale = scale;
+    coarse.binned = scale != 0.0f;
+    const FineBin fine = fine_bins(gm, scale, binned);
+    const bool by_fine = !COUNT && binned;
+    auto keep = [&](float v) {
+        return (by_fine ? fine(v) : rec_bin(coarse, v)) <= bstar && !(static_cast<double>(v) - dgm < dead);
+    };
+    {
+        bool is_cand[kSmPer];
+        uint16_t id[kSmPer];
+#pragma unroll
+        for (uint32_t q = 0; q < kSmPer; ++q) {
+            const uint32_t i = tid + NT * q;
+            is_cand[q] = live[q] && i % parts == part && keep(wm[q]);
+            id[q] = static_cast<uint16_t>(i);
+        }
+        wave_put_n(is_cand, id, &sh.c.misc[3], sh.cwave, kSampleMaxWaves);
+    }
+    __syncthreads();
+    const uint32_t ncw = sh.c.misc[3];
+    for_entries(sh.cwave, ncw, b.rec_shift, b.vocab, lg, [&](auto& v, auto& r, auto& in) {
+        constexpr uint32_t N = sizeof(in) / sizeof(in[0]);
+        bool kp[N];
+        uint64_t kk[N];
+#pragma unroll
+        for (uint32_t q = 0; q < N; ++q) {
+            kp[q] = in[q] && keep(v[q]);
+            if constexpr (COUNT) {
+                if (kp[q]) atomicAdd(&sh.hist[fine(v[q])], 1u);
+            } else {
+                kk[q] = kp[q] ? rank_key(v[q], r[q]) : 0ull;
+            }
+        }
+        if constexpr (!COUNT) wave_put_n(kp, kk, &sh.c.misc[4], sh.keys, kPartCap);
+    });
+    __syncthreads();
+    if constexpr (COUNT) {
+        for (uint32_t i = tid; i < kFineBins; i += NT)
+            if (sh.hist[i] != 0) atomicAdd(&st.hist[i], sh.hist[i]);
+    } else {
+        const uint32_t n = sh.c.misc[4];
+        // a part that overflows makes the row's list one: the finish then gathers it again
+        if (tid == 0 && n != 0) sh.base = atomicAdd(&st.n, n <= kPartCap ? n : kWideCap + 1);
+        __syncthreads();
+        if (n == 0 || n > kPartCap) return;
+        uint64_t* keys = b.keys + static_cast<size_t>(j) * b.npad;
+        for (uint32_t i = tid; i < n; i += NT)
+            if (sh.base + i < kWideCap) keys[sh.base + i] = sh.keys[i];
+    }
+}
+
+struct WideShared {
+    union {
+        uint64_t cand[kWideCap];  // the row's list
+        struct {
+            double e[kWideMax], q[kWideMax];  // then the shortlist's running sums
+        } pre;
+        LongFinishShared fin;
+    } u;
+    uint64_t sorted[kWideMax];
+    union {
+        uint16_t cwave[kSampleMaxWaves];  // candidate records, when the list is gathered again
+        uint16_t order[kWideCap];         // then the list by fine bin
+    } o;
+    uint32_t hist[kFineBins];
+    uint32_t wsum[16], big, cut, pick;
+    TopScratch t;
+    SelCommon c;
+};
+static_assert(sizeof(WideShared) <= 160 * 1024, "one block per CU");
+
+// The list of a row whose filters found more than kWideCap entries: the fine bins up to the want-th
+// entry's, or where those overflow too, the ranks from the want-th up. Returns its length; sh.hist
+// holds its inclusive fine counts (at least over the list's bins).
+__device__ __noinline__ uint32_t wide_regather(const LongBufs& b, const twd_row_params& p, uint32_t row, float gm,
+                                               const FineBin& fine, uint32_t want, WideShared& sh) {
+    constexpr int NT = kLongThreads;
+    const int tid = threadIdx.x;
+    const uint32_t W = b.waves;
+    const size_t o = static_cast<size_t>(row) * W;
+    const float* lg = b.logits + static_cast<size_t>(row) * b.stride;
+    const double dgm = static_cast<double>(gm), dead = wide_dead(p);
+    auto alive = [&](float v) { return !(static_cast<double>(v) - dgm < dead); };
+    auto list = [&](uint32_t bound) {  // records with an entry in a fine bin <= bound
+        if (tid == 0) sh.c.misc[3] = sh.c.misc[4] = 0;
+        __syncthreads();
+        for (uint32_t i0 = 0; i0 < W; i0 += NT) {
+            const uint32_t i = i0 + tid;
+            const float m = i < W ? b.st.max[o + i] : -INFINITY;
+            bool c[1] = {i < W && fine(m) <= bound && alive(m)};
+            uint16_t id[1] = {static_cast<uint16_t>(i)};
+            wave_put_n(c, id, &sh.c.misc[3], sh.o.cwave, kSampleMaxWaves);
+        }
+        __syncthreads();
+    };
+    for (uint32_t i = tid; i < kFineBins; i += NT) sh.hist[i] = 0;
+    list(kFineBins - 1);
+    for_entries(sh.o.cwave, sh.c.misc[3], b.rec_shift, b.vocab, lg, [&](auto& v, auto&, auto& in) {
+        constexpr uint32_t N = sizeof(in) / sizeof(in[0]);
+#pragma unroll
+        for (uint32_t q = 0; q < N; ++q)
+            if (in[q] && alive(v[q])) atomicAdd(&sh.hist[fine(v[q])], 1u);
+    });
+    __syncthreads();
+    fine_scan(sh.hist, sh.wsum);
+    const uint32_t t = fine_bound(sh.hist, want, &sh.big);
+    uint32_t n = sh.hist[t];
+    list(t);
+    auto gather = [&](uint64_t thr) {
+        for_entries(sh.o.cwave, sh.c.misc[3], b.rec_shift, b.vocab, lg, [&](auto& v, auto& r, auto& in) {
+            constexpr uint32_t N = sizeof(in) / sizeof(in[0]);
+            bool kp[N];
+            uint64_t kk[N];
+#pragma unroll
+            for (uint32_t q = 0; q < N; ++q) {
+                kk[q] = in[q] && fine(v[q]) <= t && alive(v[q]) ? rank_key(v[q], r[q]) : 0ull;
+                kp[q] = kk[q] != 0 && kk[q] >= thr;
+            }
+            wave_put_n(kp, kk, &sh.c.misc[4], sh.u.cand, kWideCap);
+        });
+        __syncthreads();
+    };
+    if (n <= kWideCap) {
+        gather(0);
+        return n;
+    }
+    const uint32_t nent = sh.c.misc[3] << b.rec_shift, rmask = (1u << b.rec_shift) - 1u;
+    auto key_at = [&](int e) -> uint64_t {
+        const uint32_t f = static_cast<uint32_t>(e) * NT + static_cast<uint32_t>(tid);
+        uint32_t r = 0xFFFFFFFFu;
+        if (f < nent) r = (static_cast<uint32_t>(sh.o.cwave[f >> b.rec_shift]) << b.rec_shift) + (f & rmask);
+        const float v = lg[r < b.vocab ? r : 0u];
+        return r < b.vocab && fine(v) <= t && alive(v) ? rank_key(v, r) : 0ull;
+    };
+    const uint64_t thr = block_select<NT, 0>(key_at, static_cast<int>((nent + NT - 1) / NT), want, sh.t.hist, sh.c);
+    __syncthreads();
+    gather(thr);
+    n = want;
+    for (uint32_t i = tid; i < kFineBins; i += NT) sh.hist[i] = 0;
+    __syncthreads();
+    for (uint32_t i = tid; i < n; i += NT) atomicAdd(&sh.hist[fine(rank_value(sh.u.cand[i]))], 1u);
+    __syncthreads();
+    fine_scan(sh.hist, sh.wsum);
+    return n;
+}
+
+__global__ __launch_bounds__(kLongThreads) void wide_finish_kernel(LongArgs args_by_value, LongBufs b) {
+    constexpr int NT = kLongThreads;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    WideShared& sh = *reinterpret_cast<WideShared*>(smem_raw);
+    const LongArgs& args = TWD_LONG_ARGS(args_by_value);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t j = blockIdx.x;
+    const uint32_t row = args.row[j];
+    const twd_row_params p = args.p[j];
+    const uint32_t want = min(static_cast<uint32_t>(p.top_k), b.vocab);  // <= kWideMax
+    WideState& st = b.wide[j];
+    const double total = st.total;
+    const float gm = st.gm, scale = st.scale;
+    const bool degenerate = st.degenerate != 0;
+    uint32_t n = st.n;
+    const uint64_t* list = b.keys + static_cast<size_t>(j) * b.npad;
+    __syncthreads();  // every thread has read the state
+    if (tid == 0) st.n = 0;
+    if (wide_needs_bins(want, b.waves))
+        for (uint32_t i = tid; i < kFineBins; i += NT) st.hist[i] = 0;
+    if (degenerate) {
+        if (tid == 0) b.tokens[row] = TWD_TOKEN_DEGENERATE;
+        return;
+    }
+    const FineBin fine = fine_bins(gm, scale, wide_needs_bins(want, b.waves));
+    const double dgm = static_cast<double>(gm);
+    if (n <= kWideCap) {
+        for (uint32_t i = tid; i < kFineBins; i += NT) sh.hist[i] = 0;
+        __syncthreads();
+        for (uint32_t i = tid; i < n; i += NT) {
+            const uint64_t k = list[i];
+            sh.u.cand[i] = k;
+            atomicAdd(&sh.hist[fine(rank_value(k))], 1u);
+        }
+        __syncthreads();
+        fine_scan(sh.hist, sh.wsum);
+    } else {
+        n = wide_regather(b, p, row, gm, fine, want, sh);
+    }
+
+    // ---- sorted[0 .. nl): the shortlist's live entries in descending order
+    const uint32_t nl = min(n, want);
+    if (tid == 0) sh.big = 0;
+    __syncthreads();
+    uint32_t lo[2];  // the starts of this thread's two bins
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const uint32_t i = 2 * tid + q;
+        lo[q] = i == 0 ? 0u : sh.hist[i - 1];
+        if (lo[q] < nl && sh.hist[i] - lo[q] > kWideBucket) sh.big = 1;  // every writer writes 1
+    }
+    __syncthreads();
+    if (sh.big == 0) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) sh.hist[2 * tid + q] = lo[q];
+        __syncthreads();
+        for (uint32_t i = tid; i < n; i += NT)
+            sh.o.order[atomicAdd(&sh.hist[fine(rank_value(sh.u.cand[i]))], 1u)] = static_cast<uint16_t>(i);
+        __syncthreads();  // hist[b] is bin b's end again
+        for (uint32_t i = tid; i < n; i += NT) {
+            const uint64_t k = sh.u.cand[i];
+            const uint32_t bin = fine(rank_value(k));
+            const uint32_t s0 = bin == 0 ? 0u : sh.hist[bin - 1], s1 = sh.hist[bin];
+            if (s0 >= nl) continue;
+            uint32_t at = s0;
+            for (uint32_t s = s0; s < s1; ++s) at += sh.u.cand[sh.o.order[s]] > k ? 1u : 0u;
+            if (at < nl) sh.sorted[at] = k;
+        }
+    } else {
+        uint32_t len = 2;
+        while (len < n) len <<= 1;  // <= kWideCap
+        for (uint32_t i = n + tid; i < len; i += NT) sh.u.cand[i] = 0ull;
+        __syncthreads();
+        for (uint32_t k = 2; k <= len; k <<= 1) bitonic_tile_steps(sh.u.cand, len, 0, k, k >> 1);
+        for (uint32_t i = tid; i < nl; i += NT) sh.sorted[i] = sh.u.cand[i];
+    }
+    __syncthreads();
+
+    // ---- steps 5-7: running sums of the terms (sampling.cpp:145,157), `tpt` consecutive per thread
+    const double td = static_cast<double>(p.temperature), pp = static_cast<double>(p.top_p);
+    const bool topp = p.top_p < 1.0f;
+    constexpr uint32_t kTpt = kWideMax / NT;
+    const uint32_t tpt = (want + NT - 1) / NT, i0 = tid * tpt;
+    double pe[kTpt], pq[kTpt], se = 0.0, sq = 0.0;
+#pragma unroll
+    for (uint32_t q = 0; q < kTpt; ++q) {
+        pe[q] = pq[q] = 0.0;
+        if (q < tpt && i0 + q < nl) {
+            const double l = static_cast<double>(rank_value(sh.sorted[i0 + q]));
+            pq[q] = exp_libm((l - dgm) / td);
+            if (topp) pe[q] = exp_libm(l - dgm) / total;
+        }
+        se += pe[q];
+        sq += pq[q];
+        pe[q] = se;
+        pq[q] = sq;
+    }
+    const double we = wave_incl_scan_f64(se), wq = wave_incl_scan_f64(sq);
+    if (lane == 63) {
+        sh.c.redd[wave] = we;
+        sh.c.e[wave] = wq;
+    }
+    if (tid == 0) {
+        sh.cut = want;
+        sh.pick = want;
+    }
+    __syncthreads();
+    double ae = 0.0, aq = 0.0;  // the waves and the lanes below
+    for (int w = 0; w < wave; ++w) {
+        ae += sh.c.redd[w];
+        aq += sh.c.e[w];
+    }
+    ae += dpp_move<0x138>(0.0, we);
+    aq += dpp_move<0x138>(0.0, wq);
+#pragma unroll
+    for (uint32_t q = 0; q < kTpt; ++q)
+        if (q < tpt && i0 + q < want) {
+            sh.u.pre.e[i0 + q] = ae + pe[q];
+            sh.u.pre.q[i0 + q] = aq + pq[q];
+        }
+    __syncthreads();
+    // the first prefix that reaches x (one writer where the prefixes rise; where rounding makes
+    // them fall by an ulp, x lies within the margin)
+    auto first = [&](const double* pre, uint32_t lim, double x, uint32_t* out) {
+        for (uint32_t i = tid; i < lim; i += NT)
+            if (pre[i] >= x && (i == 0 || pre[i - 1] < x)) atomicMin(out, i);
+        __syncthreads();
+        return *out;
+    };
+    bool ok = true;
+    uint32_t cut = want;
+    if (topp) {
+        const double tc = kSumTol + total_tol(b.vocab);
+        const uint32_t i = first(sh.u.pre.e, want, pp, &sh.cut);
+        if (i < want) {
+            cut = i + 1;
+            ok = sh.u.pre.e[i] >= pp * (1.0 + tc) && (i == 0 || sh.u.pre.e[i - 1] < pp * (1.0 - tc));
+        } else {
+            ok = sh.u.pre.e[want - 1] < pp * (1.0 - tc);
+        }
+    }
+    const double r = static_cast<double>(p.uniform) * sh.u.pre.q[cut - 1];
+    const uint32_t pick = first(sh.u.pre.q, cut, r, &sh.pick);
+    if (pick < cut)
+        ok = ok && sh.u.pre.q[pick] >= r * (1.0 + kSumTol) &&
+             (pick == 0 || sh.u.pre.q[pick - 1] < r * (1.0 - kSumTol));
+    else
+        ok = false;
+    if (ok && pick < nl) {
+        if (tid == 0) b.tokens[row] = rank_index(sh.sorted[pick]);
+        return;
+    }
+    // within the margin (the same in every thread): the reference's own sums, from memory. Dead
+    // entries stand in as ranks of -inf, whose terms are 0.
+    uint64_t* keys = b.keys + static_cast<size_t>(j) * b.npad;
+    for (uint32_t i = tid; i < want; i += NT) keys[i] = i < nl ? sh.sorted[i] : rank_key(-INFINITY, 0);
+    __syncthreads();
+    long_finish_row(args, b, j, gm, total, sh.u.fin);
 }
 
 // ---- the wave-record path for logits that are already in memory ---------------------------------
@@ -1062,6 +1577,7 @@ void long_free(LongScratch* l) {
     (void)hipFree(l->len);
     (void)hipFree(l->gmax);
     (void)hipFree(l->total);
+    (void)hipFree(l->wide);
     *l = LongScratch{};
 }
 
@@ -1078,6 +1594,9 @@ int long_reserve(LongScratch* l, uint32_t rows, uint64_t npad) {
     if (e == hipSuccess) e = hipMalloc(&l->len, r * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMalloc(&l->gmax, r * sizeof(float));
     if (e == hipSuccess) e = hipMalloc(&l->total, r * sizeof(double));
+    if (e == hipSuccess) e = hipMalloc(&l->wide, r * sizeof(WideState));
+    if (e == hipSuccess) e = hipMemset(l->wide, 0, r * sizeof(WideState));
+    if (e == hipSuccess) e = hipDeviceSynchronize();  // the call's stream need not follow the memset's
     if (e != hipSuccess) {
         long_free(l);
         return hip_fail(e, "allocating the long-shortlist scratch");
@@ -1091,19 +1610,21 @@ int long_reserve(LongScratch* l, uint32_t rows, uint64_t npad) {
 int launch_long(LongScratch* lng, const SampleStats& st, uint32_t waves, uint32_t rec_rows, const float* logits,
                 uint64_t stride, uint32_t vocab, uint32_t rows, const twd_row_params* params, uint32_t* tokens,
                 hipStream_t stream) {
-    LongArgs a{};
+    LongArgs a{}, w{};  // shortlists past kWideMax, and up to it
     for (uint32_t r = 0; r < rows; ++r) {
         if (!long_row(params[r], vocab)) continue;
-        a.row[a.n] = r;
-        a.p[a.n] = params[r];
-        ++a.n;
+        LongArgs& x = std::min(static_cast<uint32_t>(params[r].top_k), vocab) <= kWideMax ? w : a;
+        x.row[x.n] = r;
+        x.p[x.n] = params[r];
+        ++x.n;
     }
-    if (a.n == 0) return TWD_OK;
+    if (a.n == 0 && w.n == 0) return TWD_OK;
     if (!lng) return fail(TWD_E_INVALID, "top_k > 256 needs a selector's scratch (twd_select)");
     if (waves == 0 || waves > kSampleMaxWaves) return fail(TWD_E_INVALID, "long shortlist: wave records out of range");
-    uint64_t npad = 1;
-    while (npad < vocab) npad <<= 1;
-    int rc = long_reserve(lng, a.n, npad);
+    uint64_t npad = kWideCap;
+    if (a.n != 0)
+        while (npad < vocab) npad <<= 1;
+    int rc = long_reserve(lng, std::max(a.n, w.n), npad);
     if (rc) return rc;
     LongBufs b{};
     b.logits = logits;
@@ -1118,7 +1639,25 @@ int launch_long(LongScratch* lng, const SampleStats& st, uint32_t waves, uint32_
     b.len = lng->len;
     b.gmax = lng->gmax;
     b.total = lng->total;
+    b.wide = lng->wide;
     b.tokens = tokens;
+    if (w.n != 0) {
+        // enough parts to spread the rows' entries over the chip, few enough that their own passes
+        // over the records stay a small part of the work
+        const uint32_t parts = std::min(32u, std::max(4u, 256u / w.n));
+        bool bins = false;
+        for (uint32_t j = 0; j < w.n; ++j)
+            bins |= wide_needs_bins(std::min(static_cast<uint32_t>(w.p[j].top_k), vocab), waves);
+        if (bins) {
+            wide_filter_kernel<true><<<dim3(parts, w.n), kLongThreads, sizeof(WideFilterShared), stream>>>(w, b);
+            TWD_HIP(hipGetLastError());
+        }
+        wide_filter_kernel<false><<<dim3(parts, w.n), kLongThreads, sizeof(WideFilterShared), stream>>>(w, b);
+        TWD_HIP(hipGetLastError());
+        wide_finish_kernel<<<w.n, kLongThreads, sizeof(WideShared), stream>>>(w, b);
+        TWD_HIP(hipGetLastError());
+    }
+    if (a.n == 0) return TWD_OK;
     long_gather_kernel<<<a.n, kLongThreads, sizeof(LongGatherShared), stream>>>(a, b);
     TWD_HIP(hipGetLastError());
     const uint32_t tile = static_cast<uint32_t>(std::min<uint64_t>(npad, kSortTile));
@@ -1164,6 +1703,18 @@ int enable_select_kernels() {
                                       hipFuncAttributeMaxDynamicSharedMemorySize,
                                       static_cast<int>(sizeof(LongGatherShared)));
         if (err == hipSuccess)
+            err = hipFuncSetAttribute(reinterpret_cast<const void*>(wide_filter_kernel<false>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      static_cast<int>(sizeof(WideFilterShared)));
+        if (err == hipSuccess)
+            err = hipFuncSetAttribute(reinterpret_cast<const void*>(wide_filter_kernel<true>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      static_cast<int>(sizeof(WideFilterShared)));
+        if (err == hipSuccess)
+            err = hipFuncSetAttribute(reinterpret_cast<const void*>(wide_finish_kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      static_cast<int>(sizeof(WideShared)));
+        if (err == hipSuccess)
             err = hipFuncSetAttribute(reinterpret_cast<const void*>(long_sort_tile_kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize,
                                       static_cast<int>(kSortTile * sizeof(uint64_t)));
@@ -1190,13 +1741,14 @@ int launch_select(const SelectScratch& s, float* logits, uint32_t vocab, uint32_
     a.rows = rows;
     a.parts = parts;
     a.penalty_only = penalty_only ? 1u : 0u;
-    bool any_long = false;
+    bool any_long = false, any_short = false;  // any_short: a row that the merge finishes
     for (uint32_t r = 0; r < rows; ++r) {
         const twd_row_params& p = params[r];
         if (p.repetition_penalty != 1.0f && p.history_len > 0 && !history)
             return fail(TWD_E_INVALID, "null history with a non-empty history_len");
         a.p[r] = p;
         any_long |= !penalty_only && long_row(p, vocab);
+        any_short |= !long_row(p, vocab);
     }
     const uint32_t waves = (vocab + kSampleWaveRows - 1) / kSampleWaveRows;
     const bool have_records = s.wkey != nullptr && waves <= s.wave_cap && waves <= kSampleMaxWaves;
@@ -1222,7 +1774,7 @@ int launch_select(const SelectScratch& s, float* logits, uint32_t vocab, uint32_
             penalty_hash_kernel<<<rows, kPhThreads, 0, stream>>>(a, pb);
             TWD_HIP(hipGetLastError());
         }
-        const bool aux = rows <= kAuxMaxRows;
+        const bool aux = rows <= kAuxMaxRows && any_short;
         const SampleStats st{s.wkey, s.wsum, s.wmax, aux ? s.waux : nullptr, __builtin_nanf("")};  // no cap
         WaveStatsBufs wb{logits, stride, vocab, waves,
                          (reinterpret_cast<uintptr_t>(logits) & 15) == 0 && (stride & 3) == 0 ? 1u : 0u, st};
@@ -1239,8 +1791,10 @@ int launch_select(const SelectScratch& s, float* logits, uint32_t vocab, uint32_
         mb.waves = waves;
         mb.st = st;
         mb.tokens = tokens;
-        select_sample_merge_kernel<kSampleWaveShift><<<rows, kSmThreads, sizeof(SampleMergeShared), stream>>>(a, mb);
-        TWD_HIP(hipGetLastError());
+        if (any_short) {
+            select_sample_merge_kernel<kSampleWaveShift><<<rows, kSmThreads, sizeof(SampleMergeShared), stream>>>(a, mb);
+            TWD_HIP(hipGetLastError());
+        }
         return launch_long(s.lng, st, waves, kSampleWaveRows, logits, stride, vocab, rows, params, tokens, stream);
     }
     SelectBufs b{};

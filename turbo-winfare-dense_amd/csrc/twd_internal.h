@@ -456,6 +456,7 @@ struct LongScratch {
     uint32_t* len = nullptr;   // [rows] sort length
     float* gmax = nullptr;     // [rows] row max
     double* total = nullptr;   // [rows] sum of exp(l - max)
+    struct WideState* wide = nullptr;  // [rows] the state of the shorter ones (up to 4,096 entries)
     uint32_t rows_cap = 0;
     uint64_t npad_cap = 0;
 };
