@@ -510,7 +510,7 @@ __device__ __forceinline__ uint32_t wave_id() {
     return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 }
 
-// ---- M <= 16: the whole h resident in LDS, no barrier in the streaming loop --------------------
+// ---- M <= 8: the whole h resident in LDS, no barrier in the streaming loop ---------------------
 //
 // LDS holds the prepared h in A-fragment order, [m][chunk U][k-step t][kg] of 16 B, and the bias
 // A-fragment entries [super-unit P][slice kg][m] of 16 B, both over npad = nunits rounded up to
@@ -528,8 +528,8 @@ __host__ __device__ constexpr uint32_t resident_pad_units(uint32_t nunits) { ret
 // MS spreads the rows over the MFMA's 16 A rows: h row m sits in A row MS * m, so its outputs
 // land in accumulator entry i = (MS * m) % 4 of the lanes with lane / 16 = MS * m / 4. With
 // MS = 4 (M <= 4) every output is entry 0 and each group costs one scale FMA per accumulator
-// instead of four; MS = 2 (M <= 8) uses entries 0 and 2, MS = 1 (M <= 16) all four. A rows that
-// carry no h row read row 0; their outputs are never stored.
+// instead of four; MS = 2 (M <= 8) uses entries 0 and 2. A rows that carry no h row read row 0;
+// their outputs are never stored.
 //
 // NORM: the final RMSNorm as the prologue (M <= 4 with MS = 4, M <= 8 with MS = 2). Each block
 // computes the rows' mean squares itself and stages h = (x * rms) * w, which is fp32, as two bf16
@@ -543,13 +543,12 @@ __host__ __device__ constexpr uint32_t resident_pad_units(uint32_t nunits) { ret
 // Deepest head: 66 chunks, 8 rows of which fit in LDS beside the finish state.
 constexpr int kResidentWaves = 16;
 constexpr uint32_t kMaxUnits = 66;
-constexpr int kResidentRows = 16;
+constexpr int kResidentRows = 8;
 
 template <int MS, int RT, int PF, int MODE, bool NORM = false>
 __global__ __launch_bounds__(kResidentWaves * 64) void head_small_kernel(HeadArgs a) {
     static_assert(PF % 2 == 0, "the ring holds whole super-units");
-    static_assert(MS == 1 || MS == 2 || MS == 4, "rows spread over 16 MFMA rows with stride 1, 2 or 4");
-    static_assert(!NORM || MS >= 2, "the RMSNorm prologue takes two MFMA rows per h row");
+    static_assert(MS == 2 || MS == 4, "rows spread over 16 MFMA rows with stride 2 or 4");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     __shared__ EpiSharedT<kResidentWaves, kResidentRows> se;
     const uint32_t nw = __builtin_amdgcn_readfirstlane(blockDim.x >> 6);
@@ -876,8 +875,8 @@ __global__ __launch_bounds__(kResidentWaves * 64) void head_small_kernel(HeadArg
     }
 }
 
-// ---- 9 <= M <= 16 (and the RMSNorm prologue's 5 <= M <= 8): h prepared once per call, ------
-// staged through LDS by plain copies; M > 16 runs head_wide32_kernel below
+// ---- 9 <= M <= 16 (and RMSNorm prologues the resident-h kernel leaves): h prepared once per ----
+// call and streamed through LDS; M > 16 runs head_wide32_kernel below
 //
 // prep_hidden_kernel writes, once per call, the prepared h in A-fragment order,
 // hp[U][mt][t][lane] (16 B each, rows m >= M zero), and the bias A-fragment entries
@@ -1004,168 +1003,163 @@ __global__ __launch_bounds__(kHeadThreads) void prep_rmsnorm_kernel(const float*
     }
 }
 
-// Block = NW waves; wave w owns RT consecutive 16-row tiles. NMT = number of 16-wide m tiles
-// (1: this kernel serves M <= 16). A stage is one chunk (two groups). Each stage: one barrier;
-// the next chunk's prepared h copied straight from global memory into the other LDS buffer
-// (for an even chunk also the next super-unit's bias fragment); the weights of the next chunk
-// requested into the other half of a two-deep register ring. One chunk per stage keeps the LDS
-// small; measured on MI355X at V = 262144, d = 5376 against a two-chunk register-staged form:
-// M = 16 143.8 -> 136.2 us.
+// The prepared h passes through LDS in windows of kWinChunks chunks, two buffers: 16 rows (hp), then
+// the window's bias entries (hx). A window costs one wait and one barrier:
+//   1. wait until only the newest weight loads -- the ring's -- are outstanding: the window's copies,
+//      requested before them, have then landed; barrier (every wave's pieces are there, and every
+//      wave is done with the other buffer);
+//   2. request the next window into the other buffer (global_load_lds_dwordx4, no registers);
+//   3. kWinChunks chunks as in the resident-h kernel: weights through the PF-deep register ring,
+//      whose waits count only each slot's own loads, so the stream from HBM runs through the
+//      window's end.
+// The last window requests nothing, and leaves out the super-units past the padded chunk count.
 //
-// Per group step the MFMA chains of all RT x NMT accumulators run first; the scales are
-// applied (tot += t * acc) right after, while the next step's nibbles are converted.
-template <int NMT, int RT, int MODE, int NW>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(3)))
-void head_wide_kernel(HeadArgs a, const u32x4_t* __restrict__ hp, const u32x4_t* __restrict__ hx) {
-    constexpr int kVec = NMT * 4 * 64;  // 16 B A-fragment vectors per chunk
-    constexpr int kXA = NMT * 64;       // 16 B bias vectors per super-unit
-    constexpr int kCopies = kVec / 64 / NW;  // 1 KB pieces each wave copies per chunk
-    static_assert(kCopies >= 1 && kXA / 64 <= NW, "copy split");
-    // two buffers as separate arrays: each LDS read names the buffer it reads
-    __shared__ u32x4_t sA0[kVec], sA1[kVec];  // [mt][t][lane] of one chunk
-    __shared__ u32x4_t sXA0[kXA], sXA1[kXA];  // [mt][lane] of one super-unit
-    __shared__ EpiSharedT<NW> se;
+// The form it replaced waited for everything outstanding and met at a barrier at every chunk: M = 16
+// at V = 262,144, d = 5,376 138 -> 127 us, at V = 151,669, d = 3,584 60.7 -> 55.4, at V = 100,003,
+// d = 2,560 36.1 -> 31.2. With two m tiles it matches head_wide32_kernel on 17 to 32 rows and does not
+// beat it (159.6 against 156.3 us, 74.0 against 76.6): there the arithmetic is the longer part.
+constexpr uint32_t kWinChunks = 4;
+constexpr int kStreamRows = 16;
 
-    const int lane = threadIdx.x & 63;
+template <int RT, int PF, int MODE>
+__global__ __launch_bounds__(kResidentWaves * 64)
+void head_stream_kernel(HeadArgs a, const u32x4_t* __restrict__ hp, const u32x4_t* __restrict__ hx) {
+    constexpr uint32_t kVec = 256;  // 16 B A-fragment vectors per chunk: [t][lane]
+    constexpr uint32_t kXV = 64;    // 16 B bias vectors per super-unit: [lane]
+    constexpr uint32_t kHPieces = kWinChunks * kVec / 64, kXPieces = kWinChunks / 2 * kXV / 64;  // of 1 KB
+    constexpr uint32_t kBufVec = (kHPieces + kXPieces) * 64;
+    constexpr int kRing = PF * RT * 2;  // weight loads in flight at a window's end
+    static_assert(kWinChunks % PF == 0 && PF % 2 == 0, "a window is whole ring cycles of whole super-units");
+    static_assert(kRing < 64, "the wait counts to 63");
+    __shared__ u32x4_t buf[2][kBufVec];
+    __shared__ EpiSharedT<kResidentWaves, kStreamRows> se;
+
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t nw = __builtin_amdgcn_readfirstlane(blockDim.x >> 6);
     const uint32_t wave = wave_id();
-    const uint32_t tile0 = (blockIdx.x * NW + wave) * RT;
+    const uint32_t tile0 = (blockIdx.x * nw + wave) * RT;
     const uint32_t magic = vgpr_const(0x43004300u);
-    // an odd chunk count ends with hp's zero chunk; its weight loads re-read the last unit
-    const uint32_t nchunks = a.nunits + (a.nunits & 1);
+    const uint32_t npad = a.nunits + (a.nunits & 1), last = a.nunits - 1;
+    const uint32_t nwin = (npad + kWinChunks - 1) / kWinChunks;
 
     __amdgpu_buffer_rsrc_t rs[RT];
     tile_streams<RT>(a, tile0, rs);
     const uint32_t vo_w = lane * 16, vo_s = kUnitNibbleBytes + (lane & 15) * 8;
 
-    // 16 B per lane from global memory into LDS at l + 16 * lane (global_load_lds_dwordx4 with
-    // the wave's LDS base in M0). Issued by inline asm, so the compiler neither holds its LDS
-    // reads of the other buffer behind these copies nor counts them: the wait and barrier at
-    // each stage's start cover them. hp and hx hold one chunk and one super-unit past the end,
-    // so the copies need no branch.
+    // 16 B per lane from global memory into LDS at l + 16 * lane (the wave's LDS base in M0). Issued
+    // by inline asm, so the compiler neither holds its LDS reads of the other buffer behind these
+    // copies nor counts them: the wait and barrier at each window's start cover them. M0 is
+    // reserved to the compiler, which sets it next to each instruction of its own that reads it;
+    // this kernel has none, so the value left here is never read.
     auto copy16 = [&](const u32x4_t* g, u32x4_t* l) {
-        // the LDS offset of l: an address-space cast, not the low bits of the flat address
-        const uint32_t la = static_cast<uint32_t>(
-            reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) u32x4_t*)l));
-        // M0 is reserved to the compiler, which sets it next to each instruction of its own that
-        // reads it; this kernel has no such instruction, so the value left here is never read
-        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(la), "v"(g) : "memory");
+        const uint32_t la = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(
+            reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) u32x4_t*)l)));
+        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(la), "v"(vo_w), "s"(g) : "memory");
     };
-    auto chunk_copy = [&](uint32_t C, auto parity) {
-        constexpr int P = decltype(parity)::value;
-        u32x4_t* dst = P ? sA1 : sA0;
-        const u32x4_t* src = hp + static_cast<size_t>(C) * kVec;
-#pragma unroll
-        for (int it = 0; it < kCopies; ++it) {
-            const uint32_t piece = wave * kCopies + it;
-            copy16(src + piece * 64 + lane, dst + piece * 64);
-        }
-        // chunk C opens super-unit C / 2 when even; its bias buffer is (C / 2) & 1
-        if constexpr (P == 0) {
-            if (wave < static_cast<uint32_t>(kXA / 64)) {
-                copy16(hx + static_cast<size_t>(C >> 1) * kXA + wave * 64 + lane,
-                       (((C >> 1) & 1) ? sXA1 : sXA0) + wave * 64);
-            }
-        }
-    };
-    // chunk C's weights into ring slot B: the lane's 16 B of nibbles and its row's two {b, t} words
-    u32x4_t wr[2][RT];
-    u32x2_t sc[2][RT];
-    auto chunk_w = [&](uint32_t C, auto slot) {
-        constexpr int B = decltype(slot)::value;
-        const int so = static_cast<int>(min(C, a.nunits - 1) * kUnitBytes);
-#pragma unroll
-        for (int j = 0; j < RT; ++j) {
-            wr[B][j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs[j], vo_w, so, kNonTemporal));
-            sc[B][j] = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(rs[j], vo_s, so, kNonTemporal));
+    // window w's pieces, spread over the waves; hp and hx hold a window past the last chunk
+    auto copy_window = [&](uint32_t w) {
+        u32x4_t* dst = buf[w & 1];
+        for (uint32_t p = wave; p < kHPieces + kXPieces; p += nw) {
+            const u32x4_t* src = p < kHPieces ? hp + static_cast<size_t>(w) * (kWinChunks * kVec) + p * 64
+                                              : hx + static_cast<size_t>(w) * (kWinChunks / 2 * kXV) + (p - kHPieces) * 64;
+            copy16(src, dst + p * 64);
         }
     };
 
-    f32x4_t tot[RT][NMT];
+    u32x4_t wq[PF][RT];
+    u32x2_t sq[PF][RT];
+    copy_window(0);
 #pragma unroll
-    for (int j = 0; j < RT; ++j)
-#pragma unroll
-        for (int mt = 0; mt < NMT; ++mt) tot[j][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    bf16x8_t bq[2][RT][2];  // converted nibbles of the current and the next group step
-    u32x2_t sc_even[RT];    // the even chunk's {b, t} words, for the super-unit's bias MFMA
-
-    using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, 1>;
-    chunk_copy(0, I0{});
-    chunk_w(0, I0{});
-    __builtin_amdgcn_s_waitcnt(kWaitVm0);
-#pragma unroll
-    for (int j = 0; j < RT; ++j) {
-        bq[0][j][0] = nibbles_to_bf16(wr[0][j].x, magic);
-        bq[0][j][1] = nibbles_to_bf16(wr[0][j].y, magic);
+    for (int s = 0; s < PF; ++s) {
+        const uint32_t U = min(static_cast<uint32_t>(s), last);
+        load_nibbles_ordered<RT>(rs, U, vo_w, wq[s]);
+        load_scales_ordered<RT>(rs, U, vo_s, sq[s]);
     }
+    f32x4_t tot[RT][1];
+#pragma unroll
+    for (int j = 0; j < RT; ++j) tot[j][0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-    // chunk C in LDS buffer and ring slot P = C & 1
-    auto stage = [&](uint32_t C, auto parity) {
-        constexpr int P = decltype(parity)::value;
-        const u32x4_t* sA = P ? sA1 : sA0;
-        __builtin_amdgcn_s_waitcnt(kWaitVm0);  // this wave's copies of chunk C, its weights
-        __syncthreads();                        // every wave's copies; buffer P ^ 1 is free
-        chunk_copy(C + 1, std::integral_constant<int, P ^ 1>{});
-        chunk_w(C + 1, std::integral_constant<int, P ^ 1>{});
+    // chunk U0 + s, its weights in ring slot s: its A entries at h[s * kVec], and for an odd one its
+    // super-unit's bias entries at x
+    auto step = [&](const u32x4_t* h, const u32x4_t* x, uint32_t U0, auto slot, auto reload) {
+        constexpr int s = decltype(slot)::value;
+        const uint32_t U = U0 + s;
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
-            bf16x8_t av[NMT][2];
+            bf16x8_t av[2];
 #pragma unroll
-            for (int mt = 0; mt < NMT; ++mt)
-#pragma unroll
-                for (int t = 0; t < 2; ++t)
-                    av[mt][t] = __builtin_bit_cast(bf16x8_t, sA[(mt * 4 + 2 * g + t) * 64 + lane]);
-            f32x4_t acc[RT][NMT];
-#pragma unroll
-            for (int j = 0; j < RT; ++j)
-#pragma unroll
-                for (int mt = 0; mt < NMT; ++mt) {
-                    acc[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[mt][0], bq[g][j][0],
-                                                                         f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                    acc[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[mt][1], bq[g][j][1], acc[j][mt], 0, 0, 0);
-                }
-            // the next step's nibbles: this chunk's second group, or the next chunk's first
+            for (int t = 0; t < 2; ++t) av[t] = __builtin_bit_cast(bf16x8_t, h[s * kVec + (2 * g + t) * 64 + lane]);
+            f32x4_t acc[RT];
 #pragma unroll
             for (int j = 0; j < RT; ++j) {
-                const u32x4_t& nx = (g == 0) ? wr[P][j] : wr[P ^ 1][j];
-                bq[g ^ 1][j][0] = nibbles_to_bf16(g == 0 ? nx.z : nx.x, magic);
-                bq[g ^ 1][j][1] = nibbles_to_bf16(g == 0 ? nx.w : nx.y, magic);
+                const bf16x8_t b0 = nibbles_to_bf16(wq[s][j][2 * g], magic);
+                const bf16x8_t b1 = nibbles_to_bf16(wq[s][j][2 * g + 1], magic);
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[0], b0, f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[1], b1, acc[j], 0, 0, 0);
             }
 #pragma unroll
             for (int j = 0; j < RT; ++j) {
-                const float t = bf16_hi(g == 0 ? sc[P][j].x : sc[P][j].y);
+                const float t = bf16_hi(g ? sq[s][j].y : sq[s][j].x);
 #pragma unroll
-                for (int mt = 0; mt < NMT; ++mt)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) tot[j][mt][i] = fmaf(t, acc[j][mt][i], tot[j][mt][i]);
+                for (int i = 0; i < 4; ++i) tot[j][0][i] = fmaf(t, acc[j][i], tot[j][0][i]);
             }
         }
-        if constexpr (P == 0) {
-#pragma unroll
-            for (int j = 0; j < RT; ++j) sc_even[j] = sc[0][j];
+        constexpr bool kReload = decltype(reload)::value;
+        const uint32_t Un = min(U + PF, last);
+        if constexpr ((s & 1) == 0) {
+            if constexpr (kReload) load_nibbles_ordered<RT>(rs, Un, vo_w, wq[s]);
         } else {
-            // the super-unit's bias after its odd chunk: one K=32 MFMA per row tile and m tile
-            const u32x4_t* sXA = ((C >> 1) & 1) ? sXA1 : sXA0;
-            bf16x8_t xa[NMT];
-#pragma unroll
-            for (int mt = 0; mt < NMT; ++mt) xa[mt] = __builtin_bit_cast(bf16x8_t, sXA[mt * 64 + lane]);
+            // the super-unit's bias (see the resident-h kernel)
+            const bf16x8_t xa = __builtin_bit_cast(bf16x8_t, x[(s >> 1) * kXV + lane]);
 #pragma unroll
             for (int j = 0; j < RT; ++j) {
-                const u32x4_t bw = u32x4_t{sc_even[j].x, sc_even[j].y, sc[1][j].x, sc[1][j].y};
-#pragma unroll
-                for (int mt = 0; mt < NMT; ++mt)
-                    tot[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[mt], __builtin_bit_cast(bf16x8_t, bw),
-                                                                         tot[j][mt], 0, 0, 0);
+                const u32x4_t bp = u32x4_t{sq[s - 1][j].x, sq[s - 1][j].y, sq[s][j].x, sq[s][j].y};
+                tot[j][0] += __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, __builtin_bit_cast(bf16x8_t, bp),
+                                                                     f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            }
+            if constexpr (kReload) {
+                load_scales_ordered<RT>(rs, min(U - 1 + PF, last), vo_s, sq[s - 1]);
+                load_nibbles_ordered<RT>(rs, Un, vo_w, wq[s]);
+                load_scales_ordered<RT>(rs, Un, vo_s, sq[s]);
             }
         }
+        __builtin_amdgcn_sched_barrier(0);
     };
-    for (uint32_t C = 0; C < nchunks; C += 2) {
-        stage(C, I0{});
-        stage(C + 1, I1{});
+    auto arrive = [&]() {
+        __builtin_amdgcn_s_waitcnt(0x0F70 | (kRing & 15) | ((kRing >> 4) << 14));
+        __syncthreads();
+    };
+    uint32_t w = 0;
+    for (; w + 1 < nwin; ++w) {
+        arrive();
+        copy_window(w + 1);
+        const u32x4_t* h = buf[w & 1];
+#pragma unroll 1
+        for (uint32_t c = 0; c < kWinChunks; c += PF)
+            static_for<PF>([&](auto slot) {
+                step(h + c * kVec, h + kHPieces * 64 + (c >> 1) * kXV, w * kWinChunks + c, slot, std::true_type{});
+            });
     }
-    __builtin_amdgcn_s_waitcnt(kWaitVm0);  // the last (unused) copies land before LDS is reused
-    __syncthreads();
-    head_epilogue<NMT, 4, RT, MODE>(a, tot, tile0, se);
+    // the last window: its weight requests run on, clamped to the last unit, up to its last cycle
+    arrive();
+    const u32x4_t* h = buf[w & 1];
+    const uint32_t nlast = npad - w * kWinChunks;  // 2 .. kWinChunks
+    uint32_t c = 0;
+#pragma unroll 1
+    for (; c + PF < nlast; c += PF)
+        static_for<PF>([&](auto slot) {
+            step(h + c * kVec, h + kHPieces * 64 + (c >> 1) * kXV, w * kWinChunks + c, slot, std::true_type{});
+        });
+    static_for<PF / 2>([&](auto pair) {
+        constexpr int k = 2 * decltype(pair)::value;
+        if (k == 0 || c + k < nlast) {
+            const u32x4_t* hc = h + c * kVec;
+            const u32x4_t* xc = h + kHPieces * 64 + (c >> 1) * kXV;
+            step(hc, xc, w * kWinChunks + c, std::integral_constant<int, k>{}, std::false_type{});
+            step(hc, xc, w * kWinChunks + c, std::integral_constant<int, k + 1>{}, std::false_type{});
+        }
+    });
+    head_epilogue<1, 4, RT, MODE>(a, tot, tile0, se);
 }
 
 // ---- 33 <= M <= 64: 32x32x16 MFMAs, weights and h streamed into LDS two chunks ahead ----------
@@ -1595,8 +1589,6 @@ struct twd_head {
 
 namespace {
 
-// staged-h kernel (M <= 16): row tiles per wave, measured best on MI355X
-constexpr int kRT1 = 4;
 constexpr size_t kLdsBytes = 160 * 1024;
 constexpr uint32_t kCUs = 256;
 // upper bound of the resident-h kernel's static LDS (finish state, tables, square sums)
@@ -1638,7 +1630,7 @@ size_t resident_h_bytes(uint32_t lds_rows, uint32_t nunits) {
 // 19.2 -> 12.3 / 33.1 -> 13.7; V = 65,536 d = 4,096 (RT 1, 2 x 8 / 16) 36.6 -> 27.5 / 60.9 -> 29.7;
 // V = 100,003 d = 2,560 (RT 2, 2 x 7) 29.0 -> 27.1 / 42.7 -> 28.8; V = 151,669 d = 3,584 (RT 4,
 // 10) 64.3 -> 51.8 / 58.7 -> 53.8; V = 262,144 d = 5,376 unchanged. With the finish by groups and
-// h requested first, V = 32,003: 10.9 / 11.8; M = 12 26.7 -> 17.1.
+// h requested first, V = 32,003: 10.9 / 11.8.
 struct ResidentShape {
     int ms = 0, rt = 0;        // rows MS apart in the MFMA's rows, RT tiles per wave
     uint32_t nw = 0, blocks = 0;
@@ -1649,7 +1641,7 @@ struct ResidentShape {
 
 ResidentShape resident_shape(uint32_t ntiles, uint32_t nunits, uint32_t rows, bool norm, bool sample) {
     ResidentShape s;
-    s.ms = rows <= 4 ? 4 : rows <= 8 ? 2 : 1;
+    s.ms = rows <= 4 ? 4 : 2;
     s.rt = ntiles <= 16 * kCUs ? 1 : ntiles <= 32 * kCUs ? 2 : 4;
     const size_t hb = resident_h_bytes(norm ? 2 * rows : rows, nunits);
     auto bytes = [&](uint32_t nw) {  // the sample mode's occurrence counts lie past h
@@ -1667,12 +1659,10 @@ ResidentShape resident_shape(uint32_t ntiles, uint32_t nunits, uint32_t rows, bo
     s.bytes = bytes(s.nw);
     // short streams, and more blocks than CUs, finish together
     s.tree = s.rt == 1 || s.blocks > kCUs;
-    // Past eight rows the kernel is instantiated, and used, for one tile per wave only (at
-    // V = 100,003, d = 2,560 and above the staged-h kernel is as fast). Five to eight rows with
-    // the RMSNorm prologue take the staged-h kernel where it fills whole rounds too: 137.8 against
-    // 143.8 us at V = 262,144, d = 5,376, M = 5 (59.5 against 67.3 the other way at V = 151,669,
-    // d = 3,584; 68.2 against 73.2 at V = 240,003, d = 2,560).
-    s.fits = fit(s.nw, 1) && (s.ms > 1 || s.rt == 1) && !(norm && s.ms == 2 && s.rt == 4 && per_cu >= 16);
+    // Five to eight rows with the RMSNorm prologue take the streamed-h kernel where they would fill
+    // whole rounds of four tiles per wave: 133.3 against 143.8 us at V = 262,144, d = 5,376, M = 5
+    // (57.9 against 61.1 the other way at V = 151,669, d = 3,584).
+    s.fits = fit(s.nw, 1) && !(norm && s.ms == 2 && s.rt == 4 && per_cu >= 16);
     return s;
 }
 
@@ -1682,23 +1672,40 @@ hipError_t allow_smem(K kernel, size_t bytes) {
                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
 }
 
+// How the streamed-h kernel covers a head: tiles per wave as resident_shape, and blocks so that the
+// waves fill the CUs evenly, one 16-wave block where they fill them (M = 16 at V = 262,144,
+// d = 5,376: 127.1 us against 131.9 with two of 8) and two of half where 13 to 15 do (M = 9 at
+// V = 200,003, d = 1,536: 34.7 against 35.7).
+struct StreamShape {
+    int rt = 0;
+    uint32_t nw = 0, blocks = 0;
+};
+
+StreamShape stream_shape(uint32_t ntiles) {
+    StreamShape s;
+    s.rt = ntiles <= 16 * kCUs ? 1 : ntiles <= 32 * kCUs ? 2 : 4;
+    const uint32_t waves = (ntiles + s.rt - 1) / s.rt, per_cu = (waves + kCUs - 1) / kCUs;
+    s.nw = per_cu >= 16 ? 16 : per_cu > 12 ? (per_cu + 1) / 2 : std::max(per_cu, 4u);
+    s.blocks = (waves + s.nw - 1) / s.nw;
+    return s;
+}
+
 // f(kernel) for the resident-h instantiation of a shape.
 template <int MODE, bool NORM, typename F>
 void with_resident(int ms, int rt, F&& f) {
     auto by_rt = [&](auto msc) {
         constexpr int MS = decltype(msc)::value;
-        if (rt == 1) {
+        if (rt == 1)
             f(head_small_kernel<MS, 1, 4, MODE, NORM>);
-        } else if constexpr (MS > 1) {
-            if (rt == 2)
-                f(head_small_kernel<MS, 2, 4, MODE, NORM>);
-            else
-                f(head_small_kernel<MS, 4, 2, MODE, NORM>);
-        }
+        else if (rt == 2)
+            f(head_small_kernel<MS, 2, 4, MODE, NORM>);
+        else
+            f(head_small_kernel<MS, 4, 2, MODE, NORM>);
     };
-    if (ms == 4) return by_rt(std::integral_constant<int, 4>{});
-    if (NORM || MODE == kModeSample || ms == 2) return by_rt(std::integral_constant<int, 2>{});
-    if constexpr (!NORM && MODE != kModeSample) by_rt(std::integral_constant<int, 1>{});
+    if (ms == 4)
+        by_rt(std::integral_constant<int, 4>{});
+    else
+        by_rt(std::integral_constant<int, 2>{});
 }
 
 // This launch's epochs; only greedy launches count in.
@@ -1717,6 +1724,21 @@ FinishEpochs finish_epochs(twd_head* h, bool tree) {
     return ep;
 }
 
+// The streamed-h kernel, after its prep launch.
+template <int MODE>
+hipError_t launch_stream(twd_head* h, HeadArgs& a, hipStream_t stream) {
+    const StreamShape s = stream_shape(h->ntiles);
+    a.ep = finish_epochs<MODE>(h, s.rt == 1 || s.blocks > kCUs);
+    auto go = [&](auto kernel) { kernel<<<s.blocks, s.nw * 64, 0, stream>>>(a, h->hp, h->hx); };
+    if (s.rt == 1)
+        go(head_stream_kernel<1, 4, MODE>);
+    else if (s.rt == 2)
+        go(head_stream_kernel<2, 4, MODE>);
+    else
+        go(head_stream_kernel<4, 2, MODE>);
+    return hipGetLastError();
+}
+
 template <int MODE, bool NORM>
 hipError_t launch_resident(const ResidentShape& s, const HeadArgs& a, hipStream_t stream) {
     with_resident<MODE, NORM>(s.ms, s.rt, [&](auto kernel) {
@@ -1733,10 +1755,9 @@ int enable_small_kernels(uint32_t nunits) {
         if (e == hipSuccess) e = allow_smem(kernel, kLdsBytes - kResidentStaticLds);
     };
     for (int rt = 1; rt <= 4; rt *= 2) {
-        for (int ms = 1; ms <= 4; ms *= 2) {
+        for (int ms = 2; ms <= 4; ms *= 2) {
             with_resident<kModeLogits, false>(ms, rt, allow);
             with_resident<kModeGreedy, false>(ms, rt, allow);
-            if (ms == 1) continue;
             with_resident<kModeLogits, true>(ms, rt, allow);
             with_resident<kModeGreedy, true>(ms, rt, allow);
             with_resident<kModeSample, false>(ms, rt, allow);
@@ -1834,22 +1855,22 @@ int launch_head(twd_head* h, const uint16_t* hidden, uint32_t rows, float* logit
     a.drafts = drafts;
     a.n_drafts = n_drafts;
     a.vres = vres;
-    const ResidentShape shape = resident_shape(h->ntiles, h->nunits, std::min(rows, 16u), false, false);
-    const bool resident = rows <= 16 && shape.fits;
-    a.ep = finish_epochs<MODE>(h, resident && shape.tree);
-    if (resident) {
+    if (rows <= kResidentRows) {
+        const ResidentShape shape = resident_shape(h->ntiles, h->nunits, rows, false, false);  // it fits
+        a.ep = finish_epochs<MODE>(h, shape.tree);
         TWD_HIP((launch_resident<MODE, false>(shape, a, stream)));
-    } else if (rows <= 16) {
+    } else if (rows <= kStreamRows) {
         prep_hidden_kernel<1><<<padded_units(h->nunits) * 1, kHeadThreads, 0, stream>>>(hidden, rows, h->d,
                                                                                        h->hp, h->hx);
-        head_wide_kernel<1, kRT1, MODE, kHeadWaves>
-            <<<blocks_for(h->ntiles, kRT1), kHeadThreads, 0, stream>>>(a, h->hp, h->hx);
+        TWD_HIP(launch_stream<MODE>(h, a, stream));
     } else if (rows <= 32) {
+        a.ep = finish_epochs<MODE>(h, false);
         prep_hidden32_kernel<1><<<padded_units(h->nunits) * 2, kHeadThreads, 0, stream>>>(hidden, rows, h->d,
                                                                                          h->hp, h->hx);
         head_wide32_kernel<kW32Pairs, 1, kW32Waves, MODE>
             <<<blocks_for(h->ntiles, 2 * kW32Pairs, kW32Waves), kW32Waves * 64, 0, stream>>>(a, h->hp, h->hx);
     } else {
+        a.ep = finish_epochs<MODE>(h, false);
         prep_hidden32_kernel<2><<<padded_units(h->nunits) * 4, kHeadThreads, 0, stream>>>(hidden, rows, h->d,
                                                                                          h->hp, h->hx);
         head_wide32_kernel<kW32Pairs, 2, kW32Waves, MODE>
@@ -1869,7 +1890,8 @@ int launch_head_rmsnorm(twd_head* h, const float* x, const uint16_t* norm_w, flo
     if (!x || !aligned16(x)) return fail(TWD_E_INVALID, "x must be a 16-byte aligned device pointer");
     if (!norm_w || !aligned16(norm_w))
         return fail(TWD_E_INVALID, "norm_weight must be a 16-byte aligned device pointer");
-    if (rows == 0 || rows > 8) return fail(TWD_E_INVALID, "rows must be in 1..8 with the RMSNorm prologue");
+    if (rows == 0 || rows > kResidentRows)
+        return fail(TWD_E_INVALID, "rows must be in 1..8 with the RMSNorm prologue");
     if (!(eps >= 0.0f) || !std::isfinite(eps)) return fail(TWD_E_INVALID, "eps must be finite and >= 0");
     HeadArgs a{};
     a.tiled = h->tiled;
@@ -1888,8 +1910,8 @@ int launch_head_rmsnorm(twd_head* h, const float* x, const uint16_t* norm_w, flo
     a.n_drafts = n_drafts;
     a.vres = vres;
     const ResidentShape shape = resident_shape(h->ntiles, h->nunits, rows, true, false);
-    a.ep = finish_epochs<MODE>(h, shape.fits && shape.tree);
     if (shape.fits) {
+        a.ep = finish_epochs<MODE>(h, shape.tree);
         // the resident-h kernel stages the normalised rows itself, two LDS rows each
         a.x = x;
         a.norm_w = norm_w;
@@ -1900,8 +1922,7 @@ int launch_head_rmsnorm(twd_head* h, const float* x, const uint16_t* norm_w, flo
     a.fold = 1;
     prep_rmsnorm_kernel<<<padded_units(h->nunits), kHeadThreads, 0, stream>>>(x, norm_w, eps, rows, h->d,
                                                                               h->hp, h->hx);
-    head_wide_kernel<1, kRT1, MODE, kHeadWaves><<<blocks_for(h->ntiles, kRT1), kHeadThreads, 0, stream>>>(a, h->hp, h->hx);
-    TWD_HIP(hipGetLastError());
+    TWD_HIP(launch_stream<MODE>(h, a, stream));
     return TWD_OK;
 }
 
