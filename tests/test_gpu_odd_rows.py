@@ -1,0 +1,29 @@
+"""The record pass on rows that start at any float's address: odd vocabularies, odd strides and a base
+pointer off 16 bytes, with and without the record words (few rows, long shortlists). Tokens are
+compared with the oracle's sample_token on the same rows, exactly."""
+import numpy as np
+import pytest
+
+from helpers import twd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("V,pad,off", [(5003, 0, 0), (5003, 2, 1), (4099, 1, 3), (2050, 0, 2), (64, 3, 1), (63, 0, 3)])
+@pytest.mark.parametrize("rows,k", [(3, 40), (11, 40), (11, 0)])
+def test_rows_at_any_alignment(oracle, V, pad, off, rows, k):
+    import torch
+    t = twd()
+    dev = torch.device("cuda:0")
+    rng = np.random.default_rng(V + rows + k)
+    x = (3.0 * rng.standard_normal((rows, V))).astype(np.float32)
+    buf = torch.full((off + rows * (V + pad),), float("nan"), dtype=torch.float32, device=dev)
+    lg = buf[off:].view(rows, V + pad)[:, :V]
+    lg.copy_(torch.from_numpy(x))
+    sel = t.Selector(V, rows)
+    prm = [t.RowParams(0.8, 0.9 if m % 2 else 1.0, k, 1.0, float(np.float32(rng.uniform(0, 0.999))), 0.0, 0, 0)
+           for m in range(rows)]
+    got = sel.select(lg, prm).cpu().numpy().astype(np.int64) & 0xFFFFFFFF
+    sel.close()
+    want = [oracle.sample_token(x[m], p.temperature, p.top_p, p.top_k, u=p.uniform) for m, p in enumerate(prm)]
+    assert got.tolist() == want

@@ -1398,10 +1398,11 @@ void wave_stats_kernel(WaveStatsBufs b) {
     wave_records_block<NB, AUX>(b, blockIdx.x, blockIdx.y, tbl);
 }
 
-// Rows up to which the record pass also forms the record words: its blocks are then few and
-// short of work, and the words spare most merges their gather; past it the words cost the
-// pass more than the merges save (64 rows: 25.0 against 20.9 us for the pass).
+// When the record pass also forms the record words: for few rows, whose blocks are short of work,
+// and for long shortlists, whose merges they spare the most gathering (48 rows of V = 262,144, us:
+// k = 0 33.4 -> 30.8, k = 150 28.5 -> 28.0, but k = 64 24.4 -> 26.3).
 constexpr uint32_t kAuxMaxRows = 8;
+constexpr uint32_t kAuxMeanWant = 128;
 
 __global__ void verify_compare_kernel(const uint32_t* row_tokens, uint32_t rows,
                                       const uint32_t* drafts, uint32_t nd,
@@ -1742,6 +1743,7 @@ int launch_select(const SelectScratch& s, float* logits, uint32_t vocab, uint32_
     a.parts = parts;
     a.penalty_only = penalty_only ? 1u : 0u;
     bool any_long = false, any_short = false;  // any_short: a row that the merge finishes
+    uint32_t short_want = 0;                   // the sampled ones' shortlists together
     for (uint32_t r = 0; r < rows; ++r) {
         const twd_row_params& p = params[r];
         if (p.repetition_penalty != 1.0f && p.history_len > 0 && !history)
@@ -1749,6 +1751,8 @@ int launch_select(const SelectScratch& s, float* logits, uint32_t vocab, uint32_
         a.p[r] = p;
         any_long |= !penalty_only && long_row(p, vocab);
         any_short |= !long_row(p, vocab);
+        if (!long_row(p, vocab) && !(p.temperature <= 0.0f))
+            short_want += p.top_k > 0 ? static_cast<uint32_t>(p.top_k) : kMaxWant;
     }
     const uint32_t waves = (vocab + kSampleWaveRows - 1) / kSampleWaveRows;
     const bool have_records = s.wkey != nullptr && waves <= s.wave_cap && waves <= kSampleMaxWaves;
@@ -1774,10 +1778,9 @@ int launch_select(const SelectScratch& s, float* logits, uint32_t vocab, uint32_
             penalty_hash_kernel<<<rows, kPhThreads, 0, stream>>>(a, pb);
             TWD_HIP(hipGetLastError());
         }
-        const bool aux = rows <= kAuxMaxRows && any_short;
+        const bool aux = any_short && (rows <= kAuxMaxRows || short_want >= kAuxMeanWant * rows);
         const SampleStats st{s.wkey, s.wsum, s.wmax, aux ? s.waux : nullptr, __builtin_nanf("")};  // no cap
-        WaveStatsBufs wb{logits, stride, vocab, waves,
-                         (reinterpret_cast<uintptr_t>(logits) & 15) == 0 && (stride & 3) == 0 ? 1u : 0u, st};
+        WaveStatsBufs wb{logits, stride, vocab, waves, st};
         const dim3 grid((vocab + kWsEntries - 1) / kWsEntries, rows);
         if (aux)
             wave_stats_kernel<1, true><<<grid, kWsThreads, 0, stream>>>(wb);
@@ -1826,8 +1829,7 @@ int launch_select(const SelectScratch& s, float* logits, uint32_t vocab, uint32_
     }
     if (any_long) {  // their wave records from the penalised logits, then the long path
         const SampleStats st{s.wkey, s.wsum, s.wmax, nullptr, __builtin_nanf("")};  // no merge reads words
-        WaveStatsBufs wb{logits, stride, vocab, waves,
-                         (reinterpret_cast<uintptr_t>(logits) & 15) == 0 && (stride & 3) == 0 ? 1u : 0u, st};
+        WaveStatsBufs wb{logits, stride, vocab, waves, st};
         wave_stats_kernel<1, false><<<dim3((vocab + kWsEntries - 1) / kWsEntries, rows), kWsThreads, 0, stream>>>(wb);
         TWD_HIP(hipGetLastError());
         return launch_long(s.lng, st, waves, kSampleWaveRows, logits, stride, vocab, rows, params, tokens, stream);

@@ -1700,9 +1700,7 @@ int verify_draft_launches(twd_selector* sel, const float* logits, uint32_t vocab
         dsel.nsel = used;
         dsel.base = rp[0];
         for (uint32_t i = 0; i < used; ++i) dsel.u[i] = rp[i].uniform;
-        dsel.wb = WaveStatsBufs{logits, row_stride, vocab, waves,
-                                (reinterpret_cast<uintptr_t>(logits) & 15) == 0 && (row_stride & 3) == 0 ? 1u : 0u,
-                                st};
+        dsel.wb = WaveStatsBufs{logits, row_stride, vocab, waves, st};
         dsel.mb = SampleMergeBufs{logits, row_stride, vocab, waves, st, ss.verify_tokens};
     } else {
         TWD_HIP(hipEventRecord(ds.fork, s));
