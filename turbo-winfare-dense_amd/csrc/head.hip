@@ -52,6 +52,7 @@ struct HeadArgs {
     uint64_t* gctr;     // [kFinCtrWords]: grid_arrive_tree's counters
     FinishEpochs ep;
     uint32_t* tokens;
+    uint32_t* mirror;  // host memory that receives the tokens too (null: none)
     const uint32_t* drafts;
     uint32_t n_drafts;
     twd_verify_result* vres;
@@ -342,6 +343,7 @@ __device__ __forceinline__ void grid_finish(const HeadArgs& a, Epi& se) {
         const uint32_t t = rank_index(k);
         se.tok[m] = t;
         if (a.tokens) a.tokens[m] = t;
+        if (a.mirror) __hip_atomic_store(a.mirror + m, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     };
     if (a.ep.tree_epoch != 0) {
         // the 16 lanes of a row of lanes read the groups' maxima of one row m
@@ -1835,7 +1837,7 @@ int head_repack(twd_head* h, const uint8_t* wsb_dev, hipStream_t stream) {
 template <int MODE>
 int launch_head(twd_head* h, const uint16_t* hidden, uint32_t rows, float* logits,
                 uint32_t* tokens, const uint32_t* drafts, uint32_t n_drafts,
-                twd_verify_result* vres, hipStream_t stream) {
+                twd_verify_result* vres, hipStream_t stream, uint32_t* mirror = nullptr) {
     if (!h) return fail(TWD_E_INVALID, "null head");
     if (!hidden || !aligned16(hidden)) return fail(TWD_E_INVALID, "hidden must be a 16-byte aligned device pointer");
     if (rows == 0 || rows > TWD_MAX_ROWS) return fail(TWD_E_INVALID, "rows must be in 1..64");
@@ -1852,6 +1854,7 @@ int launch_head(twd_head* h, const uint16_t* hidden, uint32_t rows, float* logit
     a.gbest = h->gbest;
     a.gctr = h->gbest + TWD_MAX_ROWS;
     a.tokens = tokens;
+    a.mirror = mirror;
     a.drafts = drafts;
     a.n_drafts = n_drafts;
     a.vres = vres;
@@ -1885,7 +1888,8 @@ int launch_head(twd_head* h, const uint16_t* hidden, uint32_t rows, float* logit
 template <int MODE>
 int launch_head_rmsnorm(twd_head* h, const float* x, const uint16_t* norm_w, float eps,
                         uint32_t rows, float* logits, uint32_t* tokens, const uint32_t* drafts,
-                        uint32_t n_drafts, twd_verify_result* vres, hipStream_t stream) {
+                        uint32_t n_drafts, twd_verify_result* vres, hipStream_t stream,
+                        uint32_t* mirror = nullptr) {
     if (!h) return fail(TWD_E_INVALID, "null head");
     if (!x || !aligned16(x)) return fail(TWD_E_INVALID, "x must be a 16-byte aligned device pointer");
     if (!norm_w || !aligned16(norm_w))
@@ -1906,6 +1910,7 @@ int launch_head_rmsnorm(twd_head* h, const float* x, const uint16_t* norm_w, flo
     a.gbest = h->gbest;
     a.gctr = h->gbest + TWD_MAX_ROWS;
     a.tokens = tokens;
+    a.mirror = mirror;
     a.drafts = drafts;
     a.n_drafts = n_drafts;
     a.vres = vres;
@@ -1946,7 +1951,8 @@ bool sample_fusable(const twd_head* h, uint32_t rows, const twd_row_params* para
 // x/norm_w/eps select the RMSNorm prologue (x != nullptr) instead of bf16 hidden rows.
 int launch_head_sample(twd_head* h, const uint16_t* hidden, const float* x, const uint16_t* norm_w,
                        float eps, uint32_t rows, const twd_row_params* params,
-                       const uint32_t* history, float* logits, uint32_t* tokens, hipStream_t stream) {
+                       const uint32_t* history, float* logits, uint32_t* tokens, hipStream_t stream,
+                       uint32_t* mirror = nullptr) {
     HeadArgs a{};
     a.tiled = h->tiled;
     a.ntiles = h->ntiles;
@@ -1980,7 +1986,7 @@ int launch_head_sample(twd_head* h, const uint16_t* hidden, const float* x, cons
     else
         TWD_HIP((launch_resident<kModeSample, false>(s, a, stream)));
     return launch_sample_merge(h->stats, s.blocks * s.nw, static_cast<uint32_t>(s.rt) * kTileRows, logits, h->vocab,
-                               rows, params, tokens, h->sel->scratch.lng, stream);
+                               rows, params, tokens, mirror, h->sel->scratch.lng, stream);
 }
 
 // Runs one call's launches with the head's cross-stream ordering around them.
@@ -1995,9 +2001,56 @@ int ordered(twd_head* h, void* stream, F&& launches) {
     return rc ? rc : rc2;
 }
 
+// twd_head_sample and twd_head_sample_rmsnorm (in.x set). mirror, mirrored: see head_sample_row.
+int head_sample(twd_head* h, const HeadRow& in, uint32_t rows, const twd_row_params* params, const uint32_t* history,
+                float* logits, uint32_t* tokens, uint32_t* mirror, bool* mirrored, void* stream) {
+    if (!logits || !tokens || !params) return fail(TWD_E_INVALID, "null logits, tokens or params");
+    return ordered(h, stream, [&](hipStream_t s) {
+        if (sample_fusable(h, rows, params, in.x != nullptr)) {
+            if (in.x) {
+                if (!aligned16(in.x)) return fail(TWD_E_INVALID, "x must be a 16-byte aligned device pointer");
+                if (!in.norm_w || !aligned16(in.norm_w))
+                    return fail(TWD_E_INVALID, "norm_weight must be a 16-byte aligned device pointer");
+                if (!(in.eps >= 0.0f) || !std::isfinite(in.eps))
+                    return fail(TWD_E_INVALID, "eps must be finite and >= 0");
+            } else if (!in.hidden || !aligned16(in.hidden)) {
+                return fail(TWD_E_INVALID, "hidden must be a 16-byte aligned device pointer");
+            }
+            if (mirrored) {  // the merge finishes every row but those of the long path
+                *mirrored = true;
+                for (uint32_t m = 0; m < rows; ++m) *mirrored &= !long_row(params[m], h->vocab);
+            }
+            return launch_head_sample(h, in.hidden, in.x, in.norm_w, in.eps, rows, params, history, logits, tokens, s,
+                                      mirror);
+        }
+        const int rc = in.x ? launch_head_rmsnorm<kModeLogits>(h, in.x, in.norm_w, in.eps, rows, logits, nullptr,
+                                                               nullptr, 0, nullptr, s)
+                            : launch_head<kModeLogits>(h, in.hidden, rows, logits, nullptr, nullptr, 0, nullptr, s);
+        if (rc) return rc;
+        return launch_select(h->sel->scratch, logits, h->vocab, rows, h->vocab, params, history, tokens, s);
+    });
+}
+
 }  // namespace
 
 namespace twd {
+int head_greedy_row(twd_head* h, const HeadRow& in, uint32_t* token, uint32_t* mirror, bool* mirrored, void* stream) {
+    *mirrored = mirror != nullptr;
+    return ordered(h, stream, [&](hipStream_t s) {
+        return in.x ? launch_head_rmsnorm<kModeGreedy>(h, in.x, in.norm_w, in.eps, 1, nullptr, token, nullptr, 0,
+                                                       nullptr, s, mirror)
+                    : launch_head<kModeGreedy>(h, in.hidden, 1, nullptr, token, nullptr, 0, nullptr, s, mirror);
+    });
+}
+
+int head_sample_row(twd_head* h, const HeadRow& in, const twd_row_params* params, const uint32_t* history,
+                    float* logits, uint32_t* token, uint32_t* mirror, bool* mirrored, void* stream) {
+    *mirrored = false;
+    const int rc = head_sample(h, in, 1, params, history, logits, token, mirror, mirrored, stream);
+    *mirrored = *mirrored && mirror != nullptr;
+    return rc;
+}
+
 int head_set_norm_weight(twd_head* h, const uint16_t* host_w, uint32_t d) {
     if (!h || !host_w || d != h->d) return fail(TWD_E_INVALID, "norm weight of the wrong length");
     if (!h->norm_w) TWD_HIP(hipMalloc(&h->norm_w, static_cast<size_t>(d) * sizeof(uint16_t)));
@@ -2132,19 +2185,8 @@ TWD_API int twd_head_sample(twd_head* h, const uint16_t* hidden, uint32_t rows,
                             const twd_row_params* params, const uint32_t* history, float* logits,
                             uint32_t* tokens, void* stream) {
     clear_error();
-    if (!logits || !tokens || !params) return fail(TWD_E_INVALID, "null logits, tokens or params");
-    return ordered(h, stream, [&](hipStream_t s) {
-        if (sample_fusable(h, rows, params, false)) {
-            if (!hidden || !aligned16(hidden))
-                return fail(TWD_E_INVALID, "hidden must be a 16-byte aligned device pointer");
-            return launch_head_sample(h, hidden, nullptr, nullptr, 0.0f, rows, params, history, logits,
-                                      tokens, s);
-        }
-        int rc = launch_head<kModeLogits>(h, hidden, rows, logits, nullptr, nullptr, 0, nullptr, s);
-        if (rc) return rc;
-        return launch_select(h->sel->scratch, logits, h->vocab, rows, h->vocab, params, history,
-                             tokens, s);
-    });
+    return head_sample(h, HeadRow{hidden, nullptr, nullptr, 0.0f}, rows, params, history, logits, tokens, nullptr,
+                       nullptr, stream);
 }
 
 TWD_API int twd_head_logits_rmsnorm(twd_head* h, const float* x, const uint16_t* norm_w, float eps,
@@ -2186,21 +2228,10 @@ TWD_API int twd_head_sample_rmsnorm(twd_head* h, const float* x, const uint16_t*
                                     const uint32_t* history, float* logits, uint32_t* tokens,
                                     void* stream) {
     clear_error();
-    if (!logits || !tokens || !params) return fail(TWD_E_INVALID, "null logits, tokens or params");
-    return ordered(h, stream, [&](hipStream_t s) {
-        if (sample_fusable(h, rows, params, true)) {
-            if (!x || !aligned16(x)) return fail(TWD_E_INVALID, "x must be a 16-byte aligned device pointer");
-            if (!norm_w || !aligned16(norm_w))
-                return fail(TWD_E_INVALID, "norm_weight must be a 16-byte aligned device pointer");
-            if (!(eps >= 0.0f) || !std::isfinite(eps)) return fail(TWD_E_INVALID, "eps must be finite and >= 0");
-            return launch_head_sample(h, nullptr, x, norm_w, eps, rows, params, history, logits, tokens, s);
-        }
-        int rc = launch_head_rmsnorm<kModeLogits>(h, x, norm_w, eps, rows, logits, nullptr, nullptr, 0,
-                                                  nullptr, s);
-        if (rc) return rc;
-        return launch_select(h->sel->scratch, logits, h->vocab, rows, h->vocab, params, history,
-                             tokens, s);
-    });
+    if (h && logits && tokens && params && !x)  // a null x is not a bf16 call
+        return fail(TWD_E_INVALID, "x must be a 16-byte aligned device pointer");
+    return head_sample(h, HeadRow{nullptr, x, norm_w, eps}, rows, params, history, logits, tokens, nullptr, nullptr,
+                       stream);
 }
 
 TWD_API void* twd_head_finish_state(const twd_head* h) {

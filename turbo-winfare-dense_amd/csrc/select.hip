@@ -1838,7 +1838,7 @@ int launch_select(const SelectScratch& s, float* logits, uint32_t vocab, uint32_
 }
 
 int launch_sample_merge(const SampleStats& st, uint32_t waves, uint32_t rec_rows, const float* logits, uint32_t vocab,
-                        uint32_t rows, const twd_row_params* params, uint32_t* tokens,
+                        uint32_t rows, const twd_row_params* params, uint32_t* tokens, uint32_t* mirror,
                         LongScratch* lng, hipStream_t stream) {
     if (waves == 0 || waves > kSampleMaxWaves) return fail(TWD_E_INVALID, "sample merge: head waves out of range");
     if (rows == 0 || rows > TWD_MAX_ROWS) return fail(TWD_E_INVALID, "sample merge: rows out of range");
@@ -1855,6 +1855,7 @@ int launch_sample_merge(const SampleStats& st, uint32_t waves, uint32_t rec_rows
     b.waves = waves;
     b.st = st;
     b.tokens = tokens;
+    b.mirror = mirror;
     auto merge = [&](auto kernel) { kernel<<<rows, kSmThreads, sizeof(SampleMergeShared), stream>>>(a, b); };
     switch (rec_rows) {
         case 16: merge(select_sample_merge_kernel<4>); break;

@@ -928,7 +928,13 @@ struct SampleMergeBufs {
     uint32_t waves;       // head waves (records per row)
     SampleStats st;
     uint32_t* tokens;
+    uint32_t* mirror;     // host memory that receives the tokens too (null: none)
 };
+
+__device__ __forceinline__ void put_token(const SampleMergeBufs& b, uint32_t row, uint32_t tok) {
+    b.tokens[row] = tok;
+    if (b.mirror) __hip_atomic_store(b.mirror + row, tok, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 struct SampleMergeShared {
     uint32_t cwave[kSmMaxCand];   // the candidate waves read whole
@@ -967,7 +973,7 @@ __device__ __forceinline__ void sample_merge_row_per(const twd_row_params& p, ui
 #pragma unroll
         for (uint32_t q = 0; q < PER; ++q) k = key[q] > k ? key[q] : k;
         k = block_max_u64<NT>(k, sh.c);
-        if (tid == 0) b.tokens[row] = rank_index(k);
+        if (tid == 0) put_token(b, row, rank_index(k));
         return;
     }
     const uint32_t want = (p.top_k > 0) ? min(static_cast<uint32_t>(p.top_k), b.vocab)
@@ -1005,7 +1011,7 @@ __device__ __forceinline__ void sample_merge_row_per(const twd_row_params& p, ui
     for (uint32_t q = 0; q < PER; ++q) nan |= wm[q] != wm[q] ? 1u : 0u;
     const RecStats rs = records_stats<false, PER>(live, wm, nan, wsum, ref, want, sh.t, sh.c, dead_distance(p));
     if (rs.degenerate) {  // sampling.cpp:116-118
-        if (tid == 0) b.tokens[row] = TWD_TOKEN_DEGENERATE;
+        if (tid == 0) put_token(b, row, TWD_TOKEN_DEGENERATE);
         return;
     }
     const float gm = rs.gm;
@@ -1107,7 +1113,7 @@ __device__ __forceinline__ void sample_merge_row_per(const twd_row_params& p, ui
 #pragma unroll
     for (int w = 0; w < NT / 64; ++w) total += sh.c.redd[w];
     if (!(total > 0.0)) {  // sampling.cpp:116-118; every thread sums the same values
-        if (tid == 0) b.tokens[row] = TWD_TOKEN_DEGENERATE;
+        if (tid == 0) put_token(b, row, TWD_TOKEN_DEGENERATE);
         return;
     }
     const uint32_t n = first + sh.c.misc[4];  // may exceed kSmCap: then only counted
@@ -1147,7 +1153,7 @@ __device__ __forceinline__ void sample_merge_row_per(const twd_row_params& p, ui
         shortlist_pad(sh.c, want);
         __syncthreads();
         const uint32_t tok = finish_sums(sh.c, want, p, RowSrc{lg, b.vocab, gm, min(n, want)});
-        if (tid == 0) b.tokens[row] = tok;
+        if (tid == 0) put_token(b, row, tok);
         return;
     } else if (n <= static_cast<uint32_t>(NT)) {
         if (static_cast<uint32_t>(tid) < n) {
@@ -1213,7 +1219,7 @@ __device__ __forceinline__ void sample_merge_row_per(const twd_row_params& p, ui
             if (nlive < want) {
                 block_sort_desc(sh.c, nlive);
                 const uint32_t tok = finish_sampled(sh.c, want, p, total, RowSrc{lg, b.vocab, gm, nlive});
-                if (tid == 0) b.tokens[row] = tok;
+                if (tid == 0) put_token(b, row, tok);
                 return;
             }
         }
@@ -1236,7 +1242,7 @@ __device__ __forceinline__ void sample_merge_row_per(const twd_row_params& p, ui
         block_sort_desc(sh.c, want);
     }
     const uint32_t tok = finish_sampled(sh.c, want, p, total, RowSrc{lg, b.vocab, gm, want});
-    if (tid == 0) b.tokens[row] = tok;
+    if (tid == 0) put_token(b, row, tok);
 }
 
 // One row of the merge: the records per thread sized to the row's record count, so that rows of

@@ -477,9 +477,10 @@ int launch_long(LongScratch* lng, const SampleStats& st, uint32_t waves, uint32_
                 hipStream_t stream);
 
 // Enqueues the merge after a sample-mode head pass over `rows` rows (params: host array), and
-// the long path for rows with top_k > 256 (lng: their scratch).
+// the long path for rows with top_k > 256 (lng: their scratch). mirror: host memory that receives
+// the merge's tokens too (null: none; the long path's rows are not mirrored).
 int launch_sample_merge(const SampleStats& st, uint32_t waves, uint32_t rec_rows, const float* logits, uint32_t vocab,
-                        uint32_t rows, const twd_row_params* params, uint32_t* tokens,
+                        uint32_t rows, const twd_row_params* params, uint32_t* tokens, uint32_t* mirror,
                         LongScratch* lng, hipStream_t stream);
 
 // ---- device scratch shared by the launch helpers ------------------------------------------------------
@@ -533,6 +534,18 @@ struct DraftScratch {
 };
 
 int draft_scratch_reserve(DraftScratch* d, uint32_t vocab, uint32_t npos);
+// One row of the decode loop: twd_head_greedy and twd_head_sample (x null: from the bf16 hidden row;
+// else their *_rmsnorm forms), with the token also written to `mirror`, pinned host memory, by the
+// kernel that finds it -- *mirrored tells whether this call's route does.
+struct HeadRow {
+    const uint16_t* hidden;
+    const float* x;
+    const uint16_t* norm_w;
+    float eps;
+};
+int head_greedy_row(twd_head* h, const HeadRow& in, uint32_t* token, uint32_t* mirror, bool* mirrored, void* stream);
+int head_sample_row(twd_head* h, const HeadRow& in, const twd_row_params* params, const uint32_t* history,
+                    float* logits, uint32_t* token, uint32_t* mirror, bool* mirrored, void* stream);
 // Gives the head a device copy of the final RMSNorm weight (bf16 [d]), freed with the head.
 int head_set_norm_weight(twd_head* h, const uint16_t* host_w, uint32_t d);
 void draft_scratch_free(DraftScratch* d);  // the buffers; the side stream stays

@@ -1701,7 +1701,7 @@ int verify_draft_launches(twd_selector* sel, const float* logits, uint32_t vocab
         dsel.base = rp[0];
         for (uint32_t i = 0; i < used; ++i) dsel.u[i] = rp[i].uniform;
         dsel.wb = WaveStatsBufs{logits, row_stride, vocab, waves, st};
-        dsel.mb = SampleMergeBufs{logits, row_stride, vocab, waves, st, ss.verify_tokens};
+        dsel.mb = SampleMergeBufs{logits, row_stride, vocab, waves, st, ss.verify_tokens, nullptr};
     } else {
         TWD_HIP(hipEventRecord(ds.fork, s));
         TWD_HIP(hipStreamWaitEvent(ds.side, ds.fork, 0));
