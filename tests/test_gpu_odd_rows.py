@@ -1,6 +1,7 @@
 """The record pass on rows that start at any float's address: odd vocabularies, odd strides and a base
 pointer off 16 bytes, with and without the record words (few rows, long shortlists). Tokens are
-compared with the oracle's sample_token on the same rows, exactly."""
+compared with the oracle's sample_token on the same rows, exactly. Also the vocabularies at which the
+merge changes the number of records that a thread holds."""
 import numpy as np
 import pytest
 
@@ -24,6 +25,24 @@ def test_rows_at_any_alignment(oracle, V, pad, off, rows, k):
     prm = [t.RowParams(0.8, 0.9 if m % 2 else 1.0, k, 1.0, float(np.float32(rng.uniform(0, 0.999))), 0.0, 0, 0)
            for m in range(rows)]
     got = sel.select(lg, prm).cpu().numpy().astype(np.int64) & 0xFFFFFFFF
+    sel.close()
+    want = [oracle.sample_token(x[m], p.temperature, p.top_p, p.top_k, u=p.uniform) for m, p in enumerate(prm)]
+    assert got.tolist() == want
+
+
+# records of 64 entries, 1,024 threads: 1, 2, 4 and 8 records a thread up to these sizes and past them
+@pytest.mark.parametrize("V", [65536, 65537, 131072, 131073, 262144, 262145])
+@pytest.mark.parametrize("rows,k", [(2, 40), (9, 0)])
+def test_rows_where_a_thread_takes_more_records(oracle, V, rows, k):
+    import torch
+    t = twd()
+    rng = np.random.default_rng(V + rows)
+    x = (3.0 * rng.standard_normal((rows, V))).astype(np.float32)
+    x[:, -1] += 9.0  # the last record's entry among the likely ones
+    prm = [t.RowParams(0.8 if m else 0.0, 0.95 if m % 2 else 1.0, k, 1.0, float(np.float32(rng.uniform(0, 0.999))),
+                       0.0, 0, 0) for m in range(rows)]
+    sel = t.Selector(V, rows)
+    got = sel.select(torch.from_numpy(x).cuda(), prm).cpu().numpy().astype(np.int64) & 0xFFFFFFFF
     sel.close()
     want = [oracle.sample_token(x[m], p.temperature, p.top_p, p.top_k, u=p.uniform) for m, p in enumerate(prm)]
     assert got.tolist() == want

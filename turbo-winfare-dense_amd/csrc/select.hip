@@ -398,7 +398,7 @@ __global__ __launch_bounds__(kMergeThreads) void select_merge_kernel(SelectArgs 
 
 // ---- after the head's sample mode (or the wave-record pass): one block per row --------------------
 // sample_merge_row (select_core.h) finishes each row from its per-64-entry records.
-template <uint32_t RSH>
+template <uint32_t RSH, uint32_t PER>
 __global__ __launch_bounds__(kSmThreads) void select_sample_merge_kernel(SelectArgs args_by_value,
                                                                          SampleMergeBufs b) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -410,8 +410,25 @@ __global__ __launch_bounds__(kSmThreads) void select_sample_merge_kernel(SelectA
     const SelectArgs& args = args_by_value;
 #endif
     const uint32_t row = blockIdx.x;
-    sample_merge_row<RSH>(args.p[row], row, b, sh);
+    sample_merge_row_per<PER, RSH>(args.p[row], row, b, sh);
 }
+
+// The merge by its record size and by the records per thread that its rows need, one kernel for each:
+// the launch is one block a row, bound by the chain of its phases and the instructions of its 16 waves
+// on one CU, so a thread that holds one record should not step through four (binning, exponential and
+// candidate test each, at every q). One kernel with a branch between the counts is no substitute: with
+// all of them in it the same rows took 0.5 to 1.5 us more. The record pass and this kernel, top_k 40,
+// one row, before (4 or 8 a thread) and after: V = 32,003 11.8 and 10.7 us, V = 100,003 10.6 and 9.9,
+// V = 262,144 (4 a thread either way) 11.5 and 11.2; 8 rows 12.2 and 11.1, 13.2 and 12.4, 13.6 and 13.5.
+using MergeKernel = void (*)(SelectArgs, SampleMergeBufs);
+template <uint32_t RSH>
+MergeKernel merge_kernel(uint32_t waves) {
+    if (waves <= kSmThreads) return select_sample_merge_kernel<RSH, 1>;
+    if (waves <= kSmThreads * 2) return select_sample_merge_kernel<RSH, 2>;
+    if (waves <= kSmThreads * (kSmPer / 2)) return select_sample_merge_kernel<RSH, kSmPer / 2>;
+    return select_sample_merge_kernel<RSH, kSmPer>;
+}
+
 
 // ---- shortlists longer than 256: top_k > 256 -------------------------------------------------------
 //
@@ -1693,12 +1710,12 @@ int enable_select_kernels() {
             err = hipFuncSetAttribute(reinterpret_cast<const void*>(select_merge_kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize,
                                       static_cast<int>(sizeof(MergeShared)));
-        for (const void* merge : {reinterpret_cast<const void*>(select_sample_merge_kernel<4>),
-                                  reinterpret_cast<const void*>(select_sample_merge_kernel<5>),
-                                  reinterpret_cast<const void*>(select_sample_merge_kernel<6>)})
-            if (err == hipSuccess)
-                err = hipFuncSetAttribute(merge, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          static_cast<int>(sizeof(SampleMergeShared)));
+        for (uint32_t waves : {1u, kSmThreads + 1u, 2 * kSmThreads + 1u, kSampleMaxWaves})
+            for (MergeKernel merge : {merge_kernel<4>(waves), merge_kernel<5>(waves), merge_kernel<6>(waves)})
+                if (err == hipSuccess)
+                    err = hipFuncSetAttribute(reinterpret_cast<const void*>(merge),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              static_cast<int>(sizeof(SampleMergeShared)));
         if (err == hipSuccess)
             err = hipFuncSetAttribute(reinterpret_cast<const void*>(long_gather_kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1795,7 +1812,7 @@ int launch_select(const SelectScratch& s, float* logits, uint32_t vocab, uint32_
         mb.st = st;
         mb.tokens = tokens;
         if (any_short) {
-            select_sample_merge_kernel<kSampleWaveShift><<<rows, kSmThreads, sizeof(SampleMergeShared), stream>>>(a, mb);
+            merge_kernel<kSampleWaveShift>(waves)<<<rows, kSmThreads, sizeof(SampleMergeShared), stream>>>(a, mb);
             TWD_HIP(hipGetLastError());
         }
         return launch_long(s.lng, st, waves, kSampleWaveRows, logits, stride, vocab, rows, params, tokens, stream);
@@ -1856,11 +1873,11 @@ int launch_sample_merge(const SampleStats& st, uint32_t waves, uint32_t rec_rows
     b.st = st;
     b.tokens = tokens;
     b.mirror = mirror;
-    auto merge = [&](auto kernel) { kernel<<<rows, kSmThreads, sizeof(SampleMergeShared), stream>>>(a, b); };
+    auto merge = [&](MergeKernel kernel) { kernel<<<rows, kSmThreads, sizeof(SampleMergeShared), stream>>>(a, b); };
     switch (rec_rows) {
-        case 16: merge(select_sample_merge_kernel<4>); break;
-        case 32: merge(select_sample_merge_kernel<5>); break;
-        case 64: merge(select_sample_merge_kernel<6>); break;
+        case 16: merge(merge_kernel<4>(waves)); break;
+        case 32: merge(merge_kernel<5>(waves)); break;
+        case 64: merge(merge_kernel<6>(waves)); break;
         default: return fail(TWD_E_INVALID, "sample merge: record rows out of range");
     }
     TWD_HIP(hipGetLastError());

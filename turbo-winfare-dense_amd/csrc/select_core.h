@@ -1245,8 +1245,9 @@ __device__ __forceinline__ void sample_merge_row_per(const twd_row_params& p, ui
     if (tid == 0) put_token(b, row, tok);
 }
 
-// One row of the merge: the records per thread sized to the row's record count, so that rows of
-// at most 4,096 records (V <= 262,144) run no code for records that do not exist.
+// One row of the merge inside another kernel (the draft verification's): the records per thread sized
+// to the row's record count, so that rows of at most 4,096 records (V <= 262,144) run no code for
+// records that do not exist. The merge's own launches choose a kernel by the count instead.
 template <uint32_t RSH>
 __device__ __forceinline__ void sample_merge_row(const twd_row_params& p, uint32_t row, const SampleMergeBufs& b,
                                                  SampleMergeShared& sh) {
