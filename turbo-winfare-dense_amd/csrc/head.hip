@@ -537,8 +537,7 @@ __host__ __device__ constexpr uint32_t resident_pad_units(uint32_t nunits) { ret
 // computes the rows' mean squares itself and stages h = (x * rms) * w, which is fp32, as two bf16
 // halves hi = bf16(h) and lo = bf16(h - hi) (|h - hi - lo| <= 2^-18 |h|) in LDS rows 2m and
 // 2m + 1, fed as A rows MS m and MS m + 1; their outputs, adjacent entries of one lane, are added
-// before the softcap. The bias term uses the group sums of hi + lo (what the MFMA rows carry), on
-// the hi rows only.
+// before the softcap. The bias term of each of the two rows uses the group sums of that row's own half.
 //
 // A block has blockDim.x / 64 <= NWM waves and owns that many times RT row tiles (resident_shape
 // picks RT and the waves).
@@ -684,22 +683,25 @@ __global__ __launch_bounds__(kResidentWaves * 64) void head_small_kernel(HeadArg
             const float xs[8] = {cur.x0.x, cur.x0.y, cur.x0.z, cur.x0.w, cur.x1.x, cur.x1.y, cur.x1.z, cur.x1.w};
             const uint32_t ws[4] = {cur.w.x, cur.w.y, cur.w.z, cur.w.w};
             u32x4_t vh, vl;
-            float sum = 0.0f, ssm = 0.0f;
+            float ssm = 0.0f;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const float h0 = xs[2 * e] * bf16_lo(ws[e]), h1 = xs[2 * e + 1] * bf16_hi(ws[e]);  // x * weight
                 vh[e] = f32x2_to_bf16(h0, h1);
                 vl[e] = f32x2_to_bf16(h0 - bf16_lo(vh[e]), h1 - bf16_hi(vh[e]));
-                // the sum of what the MFMA rows carry (hi + lo, exact in fp32), so that
-                // the bias term cancels their 128 X exactly
-                sum += bf16_lo(vh[e]) + bf16_lo(vl[e]);
-                sum += bf16_hi(vh[e]) + bf16_hi(vl[e]);
                 ssm += xs[2 * e] * xs[2 * e];
                 ssm += xs[2 * e + 1] * xs[2 * e + 1];
             }
-            sum += __shfl_xor(sum, 1);
-            sum += __shfl_xor(sum, 2);
-            sum += __shfl_xor(sum, 4);
+            // each half's group sum for the bias on its own row: a sum of bf16 values loses little or
+            // nothing in fp32, so the bias cancels the row's 128 X. (One sum of hi + lo rounds at
+            // fp32's last bit, and the MFMA's 128 X brings that back 128 s times: 4.2e-6 from the
+            // 64-bit logits for V = 185,851, d = 2,304, M = 1, and with the two sums 3.1e-6.)
+            float sumh = sum8_bf16(vh), suml = sum8_bf16(vl);
+#pragma unroll
+            for (int o = 1; o < 8; o <<= 1) {
+                sumh += __shfl_xor(sumh, o);
+                suml += __shfl_xor(suml, o);
+            }
             // a super-unit's 32 vectors are half a wave (a row holds whole super-units)
 #pragma unroll
             for (int o = 1; o < 32; o <<= 1) ssm += __shfl_xor(ssm, o);
@@ -710,10 +712,10 @@ __global__ __launch_bounds__(kResidentWaves * 64) void head_small_kernel(HeadArg
                 sH[(((2 * m + 1) * npad + U) * 4 + (c >> 2)) * 4 + (c & 3)] = prep_h(vl);
                 if ((c8 & 7) == 0) {
                     const uint32_t g = c8 >> 3;
-                    bias_slices(sum, [&](int kg) {
+                    bias_slices(sumh, [&](int kg) {
                         return xo + (((g >> 2) * 4 + kg) * lrows + 2 * m) * 4 + (g & 3);
                     });
-                    bias_slices(0.0f, [&](int kg) {
+                    bias_slices(suml, [&](int kg) {
                         return xo + (((g >> 2) * 4 + kg) * lrows + 2 * m + 1) * 4 + (g & 3);
                     });
                 }
@@ -822,18 +824,24 @@ __global__ __launch_bounds__(kResidentWaves * 64) void head_small_kernel(HeadArg
             // {b, t} words of the super-unit's four groups: the bias B fragment. The bias is added
             // super-unit by super-unit: it cancels the 128 X that the groups' FMAs bring, so the
             // running sum stays of the logit's own size (summed apart to the end, both parts grow
-            // some 17 times larger, and the logits of V = 262,144, d = 5,376 lay 9.3e-6 from the
-            // 64-bit ones; now 2.3e-6). An MFMA into tot itself chains the steps: 120.6 against
-            // 119.2 us.
+            // some 17 times larger: M = 7, V = 262,144, d = 5,376 lay 7.1e-6, 2-norm, from the 64-bit
+            // logits, and now 2.3e-6). An MFMA into tot itself rounds once less, and chains the
+            // steps: 120.6 against 119.2 us for M = 1 greedy without the norm, which keeps the sum
+            // apart; with the norm it costs nothing (120.86 and 120.91 us) and gives 3.2e-6 against 3.5e-6.
             const bf16x8_t xa = __builtin_bit_cast(bf16x8_t, xRow[(U >> 1) * 4 * lrows]);
 #pragma unroll
             for (int j = 0; j < RT; ++j) {
                 const u32x4_t bp = u32x4_t{sq[s - 1][j].x, sq[s - 1][j].y, sq[s][j].x, sq[s][j].y};
-                const f32x4_t bias = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    xa, __builtin_bit_cast(bf16x8_t, bp), f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                if constexpr (NORM) {
+                    tot[j][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, __builtin_bit_cast(bf16x8_t, bp),
+                                                                        tot[j][0], 0, 0, 0);
+                } else {
+                    const f32x4_t bias = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        xa, __builtin_bit_cast(bf16x8_t, bp), f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (i % MS == 0 || (NORM && i % MS == 1)) tot[j][0][i] += bias[i];
+                    for (int i = 0; i < 4; ++i)
+                        if (i % MS == 0) tot[j][0][i] += bias[i];
+                }
             }
             if constexpr (kReload) {
                 load_scales_ordered<RT>(rs, min(U - 1 + PF, last), vo_s, sq[s - 1]);
@@ -923,7 +931,7 @@ __global__ __launch_bounds__(kHeadThreads) void prep_hidden_kernel(const uint16_
 // x rows, bf16 weight, for rows <= 8. h is fp32, which the bf16 MFMA operands cannot hold, so
 // it is split into h_hi = bf16(h) and h_lo = bf16(h - h_hi) (|h - h_hi - h_lo| <= 2^-18 |h|),
 // placed as MFMA rows m and m + 8 of one 16-row tile; the kernel's epilogue adds row m + 8 to
-// row m (HeadArgs::fold). The bias term uses the group sums of hi + lo, on rows < 8 only.
+// row m (HeadArgs::fold). The bias term of each row uses the group sums of its own half.
 // Every block recomputes the rows' mean squares itself (M x d fp32 from L2), so the prologue
 // needs no launch of its own. Output: the hp / hx layout of prep_hidden_kernel<1>.
 __global__ __launch_bounds__(kHeadThreads) void prep_rmsnorm_kernel(const float* __restrict__ x,
@@ -984,13 +992,10 @@ __global__ __launch_bounds__(kHeadThreads) void prep_rmsnorm_kernel(const float*
             const uint32_t hi = f32x2_to_bf16(h0, h1);
             const uint32_t lo = f32x2_to_bf16(h0 - bf16_lo(hi), h1 - bf16_hi(hi));
             v[e] = lo_plane ? lo : hi;
-            // the group sum of what the MFMA rows carry, hi + lo (exact in fp32): the bias
-            // term's X must cancel the MFMA's 128 X to the last bit, or the 2^-18 gap between
-            // h and hi + lo comes back multiplied by 128 s
-            s += bf16_lo(hi) + bf16_lo(lo);
-            s += bf16_hi(hi) + bf16_hi(lo);
         }
-        if (lo_plane) s = 0.0f;  // the bias is added once, on the high rows
+        // the group sum of what this plane's MFMA row carries, for the bias on the same row (see the
+        // resident-h kernel's staging)
+        s = sum8_bf16(v);
     }
     s += __shfl_xor(s, 1);
     s += __shfl_xor(s, 2);
@@ -1111,13 +1116,14 @@ void head_stream_kernel(HeadArgs a, const u32x4_t* __restrict__ hp, const u32x4_
         if constexpr ((s & 1) == 0) {
             if constexpr (kReload) load_nibbles_ordered<RT>(rs, Un, vo_w, wq[s]);
         } else {
-            // the super-unit's bias (see the resident-h kernel)
+            // the super-unit's bias (see the resident-h kernel), by an MFMA into the running sum: 2.0e-6
+            // from the 64-bit logits, where a sum of its own, added after, gives 2.5e-6 in the same time
             const bf16x8_t xa = __builtin_bit_cast(bf16x8_t, x[(s >> 1) * kXV + lane]);
 #pragma unroll
             for (int j = 0; j < RT; ++j) {
                 const u32x4_t bp = u32x4_t{sq[s - 1][j].x, sq[s - 1][j].y, sq[s][j].x, sq[s][j].y};
-                tot[j][0] += __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, __builtin_bit_cast(bf16x8_t, bp),
-                                                                     f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                tot[j][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa, __builtin_bit_cast(bf16x8_t, bp), tot[j][0],
+                                                                    0, 0, 0);
             }
             if constexpr (kReload) {
                 load_scales_ordered<RT>(rs, min(U - 1 + PF, last), vo_s, sq[s - 1]);
