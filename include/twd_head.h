@@ -146,9 +146,10 @@ TWD_API int twd_head_verify_greedy(twd_head* head, const uint16_t* hidden_bf16, 
  * stream, or its own events), as it orders the replays themselves.
  *
  * No counterpart in the reference: the device address of that state, for diagnostics and
- * tests: 64 per-row uint64 maxima, then the arrival counter's six uint64 words
+ * tests: 64 per-row uint64 maxima, then the launch's arrival counter's six uint64 words
  * {arrivals << 32 | epoch}: the word armed for the next launch, four replay slots and the
- * fallback word. */
+ * fallback word. Launches whose blocks finish together count in by groups first, whose maxima
+ * and counters, in the same form, follow. */
 TWD_API void* twd_head_finish_state(const twd_head* head);
 
 /* ---- the same passes with the final RMSNorm as their prologue --------------------------------
