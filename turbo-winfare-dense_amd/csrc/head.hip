@@ -1057,11 +1057,14 @@ void head_stream_kernel(HeadArgs a, const u32x4_t* __restrict__ hp, const u32x4_
     // by inline asm, so the compiler neither holds its LDS reads of the other buffer behind these
     // copies nor counts them: the wait and barrier at each window's start cover them. M0 is
     // reserved to the compiler, which sets it next to each instruction of its own that reads it;
-    // this kernel has none, so the value left here is never read.
+    // this kernel has none, so the value left here is never read. The s_nop is the wait state a load
+    // into LDS needs after a scalar write of M0 (the compiler puts it there for its own; inline asm
+    // gets none): without it the load may go where the copy before it went.
     auto copy16 = [&](const u32x4_t* g, u32x4_t* l) {
         const uint32_t la = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(
             reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) u32x4_t*)l)));
-        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(la), "v"(vo_w), "s"(g) : "memory");
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(la), "v"(vo_w), "s"(g)
+                     : "memory");
     };
     // window w's pieces, spread over the waves; hp and hx hold a window past the last chunk
     auto copy_window = [&](uint32_t w) {
@@ -1343,18 +1346,19 @@ void head_wide32_kernel(HeadArgs a, const u32x4_t* __restrict__ hp, const u32x4_
     // No instruction offset: it would move the LDS address as well. Issued by inline asm,
     // invisible to the compiler's wait insertion; M0 is reserved to the compiler, which sets it
     // next to each instruction of its own that reads it, and this kernel has none, so the value
-    // left here is never read.
+    // left here is never read. The s_nop: see head_stream_kernel's copy16.
     auto dma16 = [&](const void* base, uint32_t voff, uint32_t dst) {
-        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(voff), "s"(base)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(voff), "s"(base)
                      : "memory");
     };
     // the weights stream once: non-temporal, so they do not push h out of L2
     auto dma16_nt = [&](const void* base, uint32_t voff, uint32_t dst) {
-        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(dst), "v"(voff), "s"(base)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(dst), "v"(voff),
+                     "s"(base)
                      : "memory");
     };
     auto dma4_nt = [&](const void* base, uint32_t voff, uint32_t dst) {
-        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2 nt" ::"s"(dst), "v"(voff), "s"(base)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2 nt" ::"s"(dst), "v"(voff), "s"(base)
                      : "memory");
     };
     // chunk C's h pieces into slot C & 1, with an even C also super-unit C / 2's bias pieces
