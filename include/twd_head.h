@@ -143,7 +143,11 @@ TWD_API int twd_head_verify_greedy(twd_head* head, const uint16_t* hidden_bf16, 
  * Stream capture: the head's calls (and a selector's) may be captured into a HIP graph on any
  * stream; a captured call waits for nothing and records nothing. Replays of such a graph share
  * the object's state with its other calls, so the caller orders them against those calls (one
- * stream, or its own events), as it orders the replays themselves.
+ * stream, or its own events), as it orders the replays themselves. Rows with top_k > 256 need
+ * scratch that grows with their number in one call (and the vocabulary, not top_k): inside a
+ * capture that forbids allocation it must be there already, from an eager call with as many such
+ * rows. Scratch that a captured call uses is kept until the object is destroyed, whatever later
+ * calls need.
  *
  * No counterpart in the reference: the device address of that state, for diagnostics and
  * tests: 64 per-row uint64 maxima, then the launch's arrival counter's six uint64 words

@@ -1590,35 +1590,69 @@ void scratch_free(SelectScratch* s) {
 }
 
 void long_free(LongScratch* l) {
-    (void)hipFree(l->keys);
-    (void)hipFree(l->pre);
-    (void)hipFree(l->len);
-    (void)hipFree(l->gmax);
-    (void)hipFree(l->total);
-    (void)hipFree(l->wide);
+    (void)hipFree(l->block);
+    for (uint32_t i = 0; i < l->n_retired; ++i) (void)hipFree(l->retired[i]);
     *l = LongScratch{};
 }
 
 namespace {
-int long_reserve(LongScratch* l, uint32_t rows, uint64_t npad) {
-    if (l->keys && l->rows_cap >= rows && l->npad_cap >= npad) return TWD_OK;
-    const uint32_t r = std::max(rows, l->rows_cap);
+// Zeroes device memory now, on a stream of its own: the caller's stream need not follow it and may
+// be under capture.
+hipError_t zero_now(void* p, size_t bytes) {
+    hipStream_t side = nullptr;
+    hipError_t e = hipStreamCreateWithFlags(&side, hipStreamNonBlocking);
+    if (e != hipSuccess) return e;
+    e = hipMemsetAsync(p, 0, bytes, side);
+    if (e == hipSuccess) e = hipStreamSynchronize(side);
+    (void)hipStreamDestroy(side);
+    return e;
+}
+
+int long_reserve(LongScratch* l, uint32_t rows, uint64_t npad, hipStream_t stream) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    TWD_HIP(hipStreamIsCapturing(stream, &cap));
+    const bool capturing = cap != hipStreamCaptureStatusNone;
+    if (l->block && l->rows_cap >= rows && l->npad_cap >= npad) {
+        l->captured |= capturing;
+        return TWD_OK;
+    }
+    uint32_t r = std::max(rows, l->rows_cap);
     const uint64_t n = std::max(npad, l->npad_cap);
-    long_free(l);  // waits for the device (hipFree) before the old buffers go
+    if (l->captured) {
+        if (l->n_retired == sizeof(l->retired) / sizeof(l->retired[0]))
+            return fail(TWD_E_UNSUPPORTED, "the long-shortlist scratch has outgrown too many captures");
+        if (rows > l->rows_cap) r = std::max(rows, std::min(2 * l->rows_cap, static_cast<uint32_t>(TWD_MAX_ROWS)));
+        l->retired[l->n_retired++] = l->block;
+    } else {
+        (void)hipFree(l->block);  // waits for the device before the old buffers go
+    }
+    l->block = nullptr;
+    l->rows_cap = 0;
+    l->npad_cap = 0;
+    l->captured = capturing;
     const size_t m = static_cast<size_t>(r) * n;
-    hipError_t e = hipSuccess;
-    if (e == hipSuccess) e = hipMalloc(&l->keys, m * sizeof(uint64_t));
-    if (e == hipSuccess) e = hipMalloc(&l->pre, m * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc(&l->len, r * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc(&l->gmax, r * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(&l->total, r * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc(&l->wide, r * sizeof(WideState));
-    if (e == hipSuccess) e = hipMemset(l->wide, 0, r * sizeof(WideState));
-    if (e == hipSuccess) e = hipDeviceSynchronize();  // the call's stream need not follow the memset's
+    size_t bytes = 0;
+    auto place = [&](size_t size) {
+        const size_t at = bytes;
+        bytes += (size + 255) / 256 * 256;
+        return at;
+    };
+    const size_t keys = place(m * sizeof(uint64_t)), pre = place(m * sizeof(double)), len = place(r * sizeof(uint32_t)),
+                 gmax = place(r * sizeof(float)), total = place(r * sizeof(double)), wide = place(r * sizeof(WideState));
+    hipError_t e = hipMalloc(&l->block, bytes);
+    char* const base = static_cast<char*>(l->block);
+    if (e == hipSuccess) e = zero_now(base + wide, r * sizeof(WideState));
     if (e != hipSuccess) {
-        long_free(l);
+        (void)hipFree(l->block);
+        l->block = nullptr;
         return hip_fail(e, "allocating the long-shortlist scratch");
     }
+    l->keys = reinterpret_cast<uint64_t*>(base + keys);
+    l->pre = reinterpret_cast<double*>(base + pre);
+    l->len = reinterpret_cast<uint32_t*>(base + len);
+    l->gmax = reinterpret_cast<float*>(base + gmax);
+    l->total = reinterpret_cast<double*>(base + total);
+    l->wide = reinterpret_cast<WideState*>(base + wide);
     l->rows_cap = r;
     l->npad_cap = n;
     return TWD_OK;
@@ -1640,9 +1674,8 @@ int launch_long(LongScratch* lng, const SampleStats& st, uint32_t waves, uint32_
     if (!lng) return fail(TWD_E_INVALID, "top_k > 256 needs a selector's scratch (twd_select)");
     if (waves == 0 || waves > kSampleMaxWaves) return fail(TWD_E_INVALID, "long shortlist: wave records out of range");
     uint64_t npad = kWideCap;
-    if (a.n != 0)
-        while (npad < vocab) npad <<= 1;
-    int rc = long_reserve(lng, std::max(a.n, w.n), npad);
+    while (npad < vocab) npad <<= 1;
+    const int rc = long_reserve(lng, a.n + w.n, npad, stream);
     if (rc) return rc;
     LongBufs b{};
     b.logits = logits;

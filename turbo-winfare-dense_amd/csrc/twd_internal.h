@@ -449,8 +449,12 @@ constexpr uint32_t kSampleWaveRows = 64;    // entries per record of the wave-re
 constexpr uint32_t kSampleWaveShift = 6;    // its log2
 
 // Sort and finish buffers of the rows whose shortlist is longer than kMaxWant (top_k > 256),
-// grown on demand by the calls that have such rows.
+// grown on demand by the calls that have such rows. The size follows from the vocabulary and the
+// number of such rows alone: a call with another top_k neither moves the buffers, whose addresses a
+// captured call's launches hold, nor allocates inside a capture that an earlier call was to prepare.
+// Buffers that a captured call has used are kept, after growth too, for as long as the selector.
 struct LongScratch {
+    void* block = nullptr;     // the allocation that holds all of the following
     uint64_t* keys = nullptr;  // [rows][npad] ranks to sort
     double* pre = nullptr;     // [rows][npad] running sums of the temperature weights
     uint32_t* len = nullptr;   // [rows] sort length
@@ -459,6 +463,11 @@ struct LongScratch {
     struct WideState* wide = nullptr;  // [rows] the state of the shorter ones (up to 4,096 entries)
     uint32_t rows_cap = 0;
     uint64_t npad_cap = 0;
+    bool captured = false;     // a captured call's launches hold the block
+    // outgrown blocks that such launches hold: each at least half the next one's size, so 64 rows of
+    // up to 2^19 entries (from 2^13 on) allow 12
+    void* retired[16] = {};
+    uint32_t n_retired = 0;
 };
 void long_free(LongScratch* l);
 
