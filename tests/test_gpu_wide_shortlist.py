@@ -104,3 +104,38 @@ def test_odd_temperatures_and_draws(env, oracle):
     bad[7] = np.nan
     tok = sel.select(torch.from_numpy(bad[None]).to(dev), [t.RowParams(1.0, 0.9, 700, 1.0, 0.5, 0.0, 0, 0)])
     assert int(tok.item()) & 0xFFFFFFFF == t.TOKEN_DEGENERATE
+
+
+@pytest.mark.ties
+@pytest.mark.parametrize("V", [100003, 262144, 500000])
+@pytest.mark.parametrize("k", [257, 4096])
+def test_overfull_lists(env, oracle, V, k):
+    # lists gathered again whose last fine bin is overfull too. "deep": that bin holds the whole row, in
+    # a thousandth of its range of values, so its counting by parts of the range takes three rounds;
+    # "deep_ties": the same over three values, the last round by index; "two" and "zeros": one value,
+    # -0 equal to +0
+    torch, dev, t, _ = env
+    rng = np.random.default_rng(V + k)
+
+    def row(kind):
+        if kind == "two":
+            return rng.integers(0, 2, V).astype(np.float32)
+        if kind == "zeros":
+            z = np.where(rng.random(V) < 0.5, np.float32(-0.0), np.float32(0.0)).astype(np.float32)
+            z[rng.choice(V, 100, replace=False)] = 3.5
+            return z
+        low = np.float32(1.0) + (rng.random(V).astype(np.float32) * np.float32(1e-3) if kind == "deep" else
+                                 rng.integers(0, 3, V).astype(np.float32) * np.float32(2.0 ** -23))
+        z = low.astype(np.float32)
+        z[rng.choice(V, 100, replace=False)] = -5.0
+        z[V // 3] = 600.0
+        return z
+
+    sel = t.Selector(V, 16)
+    rows, params = [], []
+    for kind in ("two", "zeros", "deep", "deep_ties"):
+        for p, temp in ((1.0, 1.7), (0.9, 0.8), (1.0, 500.0)):
+            rows.append(row(kind))
+            params.append(t.RowParams(temp, p, k, 1.0, float(np.float32(rng.uniform(0, 0.9999))), 0.0, 0, 0))
+    check((torch, dev, t, sel), oracle, rows, params, V)
+    sel.close()

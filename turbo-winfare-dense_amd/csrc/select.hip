@@ -1075,85 +1075,194 @@ struct WideShared {
         uint16_t order[kWideCap];         // then the list by fine bin
     } o;
     uint32_t hist[kFineBins];
-    uint32_t wsum[16], big, cut, pick;
+    uint32_t wsum[16], lohi[2], big, cut, pick;
     TopScratch t;
     SelCommon c;
 };
 static_assert(sizeof(WideShared) <= 160 * 1024, "one block per CU");
 
-// The list of a row whose filters found more than kWideCap entries: the fine bins up to the want-th
-// entry's, or where those overflow too, the ranks from the want-th up. Returns its length; sh.hist
-// holds its inclusive fine counts (at least over the list's bins).
-__device__ __noinline__ uint32_t wide_regather(const LongBufs& b, const twd_row_params& p, uint32_t row, float gm,
-                                               const FineBin& fine, uint32_t want, WideShared& sh) {
+// Counts into hist with a thread's two last bins held in registers: additions on one LDS address are
+// served one after another, and a row that needs counting here is mostly one of few values.
+struct Tally {
+    uint32_t* hist;
+    uint32_t b0 = 0, c0 = 0, b1 = 0, c1 = 0;
+    __device__ __forceinline__ void add(uint32_t bin) {
+        if (bin == b0) {
+            ++c0;
+        } else if (bin == b1) {
+            ++c1;
+        } else {
+            if (c1 != 0) atomicAdd(&hist[b1], c1);
+            b1 = b0;
+            c1 = c0;
+            b0 = bin;
+            c0 = 1;
+        }
+    }
+    __device__ __forceinline__ void flush() {
+        if (c0 != 0) atomicAdd(&hist[b0], c0);
+        if (c1 != 0) atomicAdd(&hist[b1], c1);
+    }
+};
+
+// The smallest float that is not dead at a row maximum gm (see dead_distance): found next to the
+// rounded sum, from where a step or two remain.
+__device__ __forceinline__ float alive_floor(double gm, double dead) {
+    if (dead == -INFINITY) return -INFINITY;
+    auto alive = [&](uint32_t k) { return !(static_cast<double>(key_float(k)) - gm < dead); };
+    uint32_t k = float_key(static_cast<float>(gm + dead));
+    const uint32_t least = float_key(-INFINITY);
+    while (!alive(k)) ++k;
+    while (k > least && alive(k - 1)) --k;
+    return key_float(k);
+}
+
+// The list of a row whose filters found more than kWideCap entries, by this block alone: the fine bins
+// up to the want-th entry's, or where the last of them overflows too (ties, mostly), the ranks from a
+// threshold up that leaves at most kWideCap. The threshold comes from counting that bin's entries by
+// parts of its range of values, and where one value alone is too many, by ranges of index. Each pass
+// reads the candidate records once, 16 entries a lane at a time, and is bound by its instructions per
+// entry on the one CU; a row of equal entries takes four. A radix select of the want-th rank read them
+// nine times, an entry at a time. The whole call, one row of V = 262,144, top_k = 300, us, with the
+// long path, with the radix select, and now: equal entries 347, 1,389, 146; two values 348, 1,464, 266.
+// Returns the list's length.
+__device__ __forceinline__ uint32_t wide_regather(const LongBufs& b, const twd_row_params& p, uint32_t row, float gm,
+                                                  const FineBin& fine, uint32_t want, WideShared& sh) {
     constexpr int NT = kLongThreads;
+    constexpr uint32_t kRunShift = 4, kRun = 1u << kRunShift;
     const int tid = threadIdx.x;
-    const uint32_t W = b.waves;
+    const uint32_t W = b.waves, rsh = b.rec_shift, vocab = b.vocab;
     const size_t o = static_cast<size_t>(row) * W;
     const float* lg = b.logits + static_cast<size_t>(row) * b.stride;
-    const double dgm = static_cast<double>(gm), dead = wide_dead(p);
-    auto alive = [&](float v) { return !(static_cast<double>(v) - dgm < dead); };
+    const float floor = alive_floor(static_cast<double>(gm), wide_dead(p));
     auto list = [&](uint32_t bound) {  // records with an entry in a fine bin <= bound
         if (tid == 0) sh.c.misc[3] = sh.c.misc[4] = 0;
         __syncthreads();
         for (uint32_t i0 = 0; i0 < W; i0 += NT) {
             const uint32_t i = i0 + tid;
             const float m = i < W ? b.st.max[o + i] : -INFINITY;
-            bool c[1] = {i < W && fine(m) <= bound && alive(m)};
+            bool c[1] = {i < W && fine(m) <= bound && m >= floor};
             uint16_t id[1] = {static_cast<uint16_t>(i)};
             wave_put_n(c, id, &sh.c.misc[3], sh.o.cwave, kSampleMaxWaves);
         }
         __syncthreads();
     };
-    for (uint32_t i = tid; i < kFineBins; i += NT) sh.hist[i] = 0;
-    list(kFineBins - 1);
-    for_entries(sh.o.cwave, sh.c.misc[3], b.rec_shift, b.vocab, lg, [&](auto& v, auto&, auto& in) {
-        constexpr uint32_t N = sizeof(in) / sizeof(in[0]);
+    // f(values, first row) over the listed records' entries, kRun consecutive ones a thread (a record
+    // holds whole runs; their rows lie in one range of index); the same trip count in every thread.
+    // Past the end NaN, which no comparison accepts.
+    auto entries = [&](auto&& f) {
+        const uint32_t esh = rsh - kRunShift, emask = (1u << esh) - 1u, ne = sh.c.misc[3] << esh;
+        for (uint32_t i0 = 0; i0 < ne; i0 += NT) {
+            const uint32_t e = i0 + tid;
+            uint32_t r0 = vocab;
+            if (e < ne) r0 = (static_cast<uint32_t>(sh.o.cwave[e >> esh]) << rsh) + ((e & emask) << kRunShift);
+            float v[kRun];
+            if (r0 + kRun <= vocab) {
 #pragma unroll
-        for (uint32_t q = 0; q < N; ++q)
-            if (in[q] && alive(v[q])) atomicAdd(&sh.hist[fine(v[q])], 1u);
-    });
-    __syncthreads();
-    fine_scan(sh.hist, sh.wsum);
-    const uint32_t t = fine_bound(sh.hist, want, &sh.big);
-    uint32_t n = sh.hist[t];
-    list(t);
-    auto gather = [&](uint64_t thr) {
-        for_entries(sh.o.cwave, sh.c.misc[3], b.rec_shift, b.vocab, lg, [&](auto& v, auto& r, auto& in) {
-            constexpr uint32_t N = sizeof(in) / sizeof(in[0]);
-            bool kp[N];
-            uint64_t kk[N];
+                for (uint32_t q = 0; q < kRun / 4; ++q) {
+                    const float4_u x = *reinterpret_cast<const float4_u*>(lg + r0 + 4 * q);
 #pragma unroll
-            for (uint32_t q = 0; q < N; ++q) {
-                kk[q] = in[q] && fine(v[q]) <= t && alive(v[q]) ? rank_key(v[q], r[q]) : 0ull;
-                kp[q] = kk[q] != 0 && kk[q] >= thr;
+                    for (uint32_t k = 0; k < 4; ++k) v[4 * q + k] = x[k];
+                }
+            } else {
+#pragma unroll
+                for (uint32_t q = 0; q < kRun; ++q) v[q] = r0 + q < vocab ? lg[r0 + q] : __builtin_nanf("");
+            }
+            f(v, r0);
+        }
+        __syncthreads();
+    };
+    // the inclusive counts by bin(value, row) of the entries from lo to hi
+    auto count = [&](float lo, float hi, auto&& bin) {
+        for (uint32_t i = tid; i < kFineBins; i += NT) sh.hist[i] = 0;
+        __syncthreads();
+        Tally tally{sh.hist};
+        entries([&](auto& v, uint32_t r) {
+#pragma unroll
+            for (uint32_t q = 0; q < kRun; ++q)
+                if (v[q] >= lo && v[q] <= hi) tally.add(bin(v[q], r + q));
+        });
+        tally.flush();
+        __syncthreads();
+        fine_scan(sh.hist, sh.wsum);
+    };
+    auto gather = [&](auto&& keep) {
+        entries([&](auto& v, uint32_t r) {
+            bool kp[kRun];
+            uint64_t kk[kRun];
+#pragma unroll
+            for (uint32_t q = 0; q < kRun; ++q) {
+                kp[q] = keep(v[q], r + q);
+                kk[q] = rank_key(v[q], r + q);
             }
             wave_put_n(kp, kk, &sh.c.misc[4], sh.u.cand, kWideCap);
         });
-        __syncthreads();
     };
+    list(kFineBins - 1);
+    count(floor, INFINITY, [&](float v, uint32_t) { return fine(v); });
+    const uint32_t t = fine_bound(sh.hist, want, &sh.big);
+    uint32_t n = sh.hist[t], above = t == 0 ? 0u : sh.hist[t - 1];  // up to the bin, and before it
+    list(t);
     if (n <= kWideCap) {
-        gather(0);
+        gather([&](float v, uint32_t) { return v >= floor && fine(v) <= t; });
         return n;
     }
-    const uint32_t nent = sh.c.misc[3] << b.rec_shift, rmask = (1u << b.rec_shift) - 1u;
-    auto key_at = [&](int e) -> uint64_t {
-        const uint32_t f = static_cast<uint32_t>(e) * NT + static_cast<uint32_t>(tid);
-        uint32_t r = 0xFFFFFFFFu;
-        if (f < nent) r = (static_cast<uint32_t>(sh.o.cwave[f >> b.rec_shift]) << b.rec_shift) + (f & rmask);
-        const float v = lg[r < b.vocab ? r : 0u];
-        return r < b.vocab && fine(v) <= t && alive(v) ? rank_key(v, r) : 0ull;
-    };
-    const uint64_t thr = block_select<NT, 0>(key_at, static_cast<int>((nent + NT - 1) / NT), want, sh.t.hist, sh.c);
+    // the range of the bin's values
+    if (tid == 0) {
+        sh.lohi[0] = 0xFFFFFFFFu;
+        sh.lohi[1] = 0u;
+    }
     __syncthreads();
-    gather(thr);
-    n = want;
-    for (uint32_t i = tid; i < kFineBins; i += NT) sh.hist[i] = 0;
+    {
+        float lo = INFINITY, hi = -INFINITY;
+        entries([&](auto& v, uint32_t) {
+#pragma unroll
+            for (uint32_t q = 0; q < kRun; ++q) {
+                const bool in = v[q] >= floor && fine(v[q]) == t;
+                lo = in ? fminf(lo, v[q]) : lo;
+                hi = in ? fmaxf(hi, v[q]) : hi;
+            }
+        });
+#pragma unroll
+        for (int msk = 1; msk < 64; msk <<= 1) {
+            lo = fminf(lo, __shfl_xor(lo, msk));
+            hi = fmaxf(hi, __shfl_xor(hi, msk));
+        }
+        if ((tid & 63) == 0) {
+            atomicMin(&sh.lohi[0], float_key(lo));
+            atomicMax(&sh.lohi[1], float_key(hi));
+        }
+    }
     __syncthreads();
-    for (uint32_t i = tid; i < n; i += NT) atomicAdd(&sh.hist[fine(rank_value(sh.u.cand[i]))], 1u);
-    __syncthreads();
-    fine_scan(sh.hist, sh.wsum);
-    return n;
+    uint32_t klo = sh.lohi[0], khi = sh.lohi[1];  // the list ends between these keys
+    for (;;) {  // at most three ranges of values (2,048 parts each), then one value
+        const bool one = klo == khi;
+        const uint32_t span = one ? vocab - 1 : khi - klo;
+        const uint32_t psh = span < kFineBins ? 0u : 21u - static_cast<uint32_t>(__builtin_clz(span));
+        if (one)
+            count(key_float(klo), key_float(khi), [&](float, uint32_t r) { return r >> psh; });
+        else
+            count(key_float(klo), key_float(khi), [&](float v, uint32_t) { return (khi - float_key(v)) >> psh; });
+        const uint32_t part = fine_bound(sh.hist, want - above, &sh.big);
+        const uint32_t before = part == 0 ? 0u : sh.hist[part - 1];
+        n = above + sh.hist[part];
+        const uint32_t end = min((part << psh) + ((1u << psh) - 1u), span);  // the part's last row or lowest key
+        __syncthreads();  // the counts are read
+        if (one) {  // above < want <= kWideMax, and a part has at most 256 rows: n < kWideCap
+            const float x = key_float(khi);
+            gather([&](float v, uint32_t r) { return v > x || (v == x && r <= end); });
+            return n;
+        }
+        const uint32_t top = khi;
+        khi = top - (part << psh);
+        klo = top - end;
+        if (n <= kWideCap) {
+            const float x = key_float(klo);
+            gather([&](float v, uint32_t) { return v >= x; });
+            return n;
+        }
+        above += before;
+    }
 }
 
 __global__ __launch_bounds__(kLongThreads) void wide_finish_kernel(LongArgs args_by_value, LongBufs b) {
@@ -1194,6 +1303,11 @@ __global__ __launch_bounds__(kLongThreads) void wide_finish_kernel(LongArgs args
         fine_scan(sh.hist, sh.wsum);
     } else {
         n = wide_regather(b, p, row, gm, fine, want, sh);
+        for (uint32_t i = tid; i < kFineBins; i += NT) sh.hist[i] = 0;
+        __syncthreads();
+        for (uint32_t i = tid; i < n; i += NT) atomicAdd(&sh.hist[fine(rank_value(sh.u.cand[i]))], 1u);
+        __syncthreads();
+        fine_scan(sh.hist, sh.wsum);
     }
 
     // ---- sorted[0 .. nl): the shortlist's live entries in descending order
