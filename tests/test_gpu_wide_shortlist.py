@@ -139,3 +139,21 @@ def test_overfull_lists(env, oracle, V, k):
             params.append(t.RowParams(temp, p, k, 1.0, float(np.float32(rng.uniform(0, 0.9999))), 0.0, 0, 0))
     check((torch, dev, t, sel), oracle, rows, params, V)
     sel.close()
+
+
+@pytest.mark.ties
+@pytest.mark.parametrize("V", [257, 300, 513, 1500, 3000, 8193])
+def test_small_vocabularies_taken_whole(env, oracle, V):
+    # shortlists that reach past the records' range, sorted by bins over the list's own: a finite range,
+    # an infinite one (-inf entries that a draw of 1 keeps), the widest finite one, equal entries
+    t = env[2]
+    rows, params = [], []
+    for kind in ("normal", "ties", "equal", "minus_inf", "outlier"):
+        for u in (0.42, 0.9999, 1.0):
+            rows.append(row_of(kind, V, V + len(rows)))
+            params.append(t.RowParams(1.1, 0.999, min(V, 4096), 1.0, u, 0.0, 0, 0))
+    wide = row_of("normal", V, 5)
+    wide[1::3] = np.finfo(np.float32).min
+    rows.append(wide)
+    params.append(t.RowParams(float("inf"), 1.0, min(V, 4096), 1.0, 0.8, 0.0, 0, 0))
+    check(env, oracle, rows, params, V)
