@@ -1750,8 +1750,7 @@ void long_free(LongScratch* l) {
 }
 
 namespace {
-// Zeroes device memory now, on a stream of its own: the caller's stream need not follow it and may
-// be under capture.
+// Zeroes device memory now, on a stream of its own: the caller's is under capture.
 hipError_t zero_now(void* p, size_t bytes) {
     hipStream_t side = nullptr;
     hipError_t e = hipStreamCreateWithFlags(&side, hipStreamNonBlocking);
@@ -1795,7 +1794,11 @@ int long_reserve(LongScratch* l, uint32_t rows, uint64_t npad, hipStream_t strea
                  gmax = place(r * sizeof(float)), total = place(r * sizeof(double)), wide = place(r * sizeof(WideState));
     hipError_t e = hipMalloc(&l->block, bytes);
     char* const base = static_cast<char*>(l->block);
-    if (e == hipSuccess) e = zero_now(base + wide, r * sizeof(WideState));
+    if (e == hipSuccess) {
+        // captured, the clear would only run with the replays, after eager calls that need it
+        e = capturing ? zero_now(base + wide, r * sizeof(WideState))
+                      : hipMemsetAsync(base + wide, 0, r * sizeof(WideState), stream);
+    }
     if (e != hipSuccess) {
         (void)hipFree(l->block);
         l->block = nullptr;
