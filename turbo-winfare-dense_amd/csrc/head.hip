@@ -1671,10 +1671,10 @@ ResidentShape resident_shape(uint32_t ntiles, uint32_t nunits, uint32_t rows, bo
     s.bytes = bytes(s.nw);
     // short streams, and more blocks than CUs, finish together
     s.tree = s.rt == 1 || s.blocks > kCUs;
-    // Five to eight rows with the RMSNorm prologue take the streamed-h kernel where they would fill
-    // whole rounds of four tiles per wave: 133.3 against 143.8 us at V = 262,144, d = 5,376, M = 5
-    // (57.9 against 61.1 the other way at V = 151,669, d = 3,584).
-    s.fits = fit(s.nw, 1) && !(norm && s.ms == 2 && s.rt == 4 && per_cu >= 16);
+    // RMSNorm rows run here wherever their two halves fit, five to eight rows too (V = 262,144, M = 5,
+    // against the prep launch and the streamed-h kernel: d = 1,024 29.2 and 37.3 us, d = 2,560 62.2 and
+    // 72.9, d = 5,376 124.8 and 134.9; seven rows of d = 5,376 no longer fit)
+    s.fits = fit(s.nw, 1);
     return s;
 }
 
