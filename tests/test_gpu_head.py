@@ -68,7 +68,7 @@ def test_layout_single_unit(torch_dev, oracle):
 
 @pytest.mark.parametrize("M", [1, 2, 4, 5, 6, 7, 8, 9, 16, 17, 33, 64])
 def test_logits_parity(torch_dev, oracle, M):
-    # M = 2..6 and M = 7, 8 run the resident-h kernel with 8 and 16 waves per block at d = 5376
+    # up to 8 rows the resident-h kernel, up to 16 the streamed-h one, past that the wide one
     V = 1000  # not a multiple of 16: the last row tile is partial
     W, S, B = oracle.gen_lm_head(100 + M, V, D)
     head = make_head(torch_dev, W, S, B, V, D, CAP)
@@ -413,7 +413,8 @@ def test_rmsnorm_logits_parity(torch_dev, oracle, d, M):
     assert [int(t) for t in tok] == [int(oracle.argmax(got[m])) for m in range(M)]
 
 
-@pytest.mark.parametrize("M", [3, 5])  # the resident-h prologue (M <= 4) and the staged one
+# 3 and 5 rows: the resident-h prologue, four and two MFMA rows apart; 8: the staged one
+@pytest.mark.parametrize("M", [3, 5, 8])
 def test_rmsnorm_verify_and_sample(torch_dev, oracle, M):
     torch, dev = torch_dev
     t = twd()

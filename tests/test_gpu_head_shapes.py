@@ -1,5 +1,6 @@
 """The resident-h head kernel's shapes: tiles per wave, waves per block and record sizes follow the
-head's size, so each side of every line of that rule runs here, at a short depth, against the
+head's size; both sides of its lines for tiles per wave and for one or two blocks a CU run here, at a
+short depth (deeper heads and more than 13 waves a CU: test_gpu_head_depth.py), against the
 oracle's scalar head (the reference kernel test's 1e-3 tolerance) and, for the tokens, against the
 oracle's selection on the device's own logits (exact)."""
 import numpy as np
@@ -15,7 +16,7 @@ D = 384  # three chunks: an odd count, so the padding chunk is there
 # to 12 waves, two blocks of half past that
 SIZES = [
     16 * 3 + 5,            # fewer tiles than one block's waves
-    49_153,                # 13 waves per CU: two blocks of 7
+    49_152, 49_153,        # 12 waves per CU | 13: two blocks of 7
     65_536, 65_537,        # one | two tiles per wave
     131_072, 131_075,      # two | four tiles per wave
 ]
