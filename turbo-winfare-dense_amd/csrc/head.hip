@@ -223,9 +223,7 @@ struct EpiSharedT {
 // finish together and are spread over kFinGroups maxima and counters, because atomics on one
 // address are served one by one: with one of each, a greedy launch took 3.8 us longer than the
 // same launch without its finish on 251 blocks (V = 32,003, d = 2,048; 12.3 against 8.5 us),
-// spread 2.3 us. Where the blocks finish apart (one block per CU with two or more tiles per wave,
-// and the wide kernels) the second level only costs its round trip (V = 262,144: M = 12 139.8
-// against 137.7 us, M = 5 126.5 against 125.4).
+// spread 2.3 us. Which launches do: finish_by_groups.
 // tot[j][mt][i] holds row r = (tile0 + j) * 16 + lane % 16 of MFMA row 16 mt + 4 (lane / 16) + i,
 // which carries h row m = (16 mt + 4 (lane / 16) + i) / MS when i is a multiple of MS (MS > 1:
 // the rows are spread over the MFMA rows, see head_small_kernel); other entries are not outputs.
@@ -1631,6 +1629,16 @@ size_t resident_h_bytes(uint32_t lds_rows, uint32_t nunits) {
     return static_cast<size_t>(lds_rows) * resident_pad_units(nunits) * (256 + 32);
 }
 
+// Blocks that finish together count in by groups (grid_arrive_tree): those of short streams -- one tile
+// per wave, or few chunks for its tiles -- and more than one a CU. Longer streams' blocks finish apart, and
+// the second level only costs its round trip. One level and groups, greedy, us: V = 65,552, M = 1 (two tiles
+// per wave) d = 256 9.2 and 8.0, 1,024 13.1 and 11.8, 2,048 18.0 and 17.3, 5,376 36.6 and 37.1; V = 131,088,
+// M = 5 (four) d = 256 11.6 and 10.3, 1,024 18.9 and 18.3, 2,048 30.0 and 30.1, 5,376 69.5 and 71.3.
+constexpr uint32_t kTreeChunks = 32;  // chunks of all tiles of a wave
+bool finish_by_groups(int rt, uint32_t blocks, uint32_t nunits) {
+    return rt == 1 || blocks > kCUs || rt * nunits <= kTreeChunks;
+}
+
 // How the resident-h kernel covers a head of `ntiles` row tiles: RT tiles per wave, nw waves per
 // block. RT is the smallest of 1, 2, 4 that leaves at most 16 waves per CU (four per SIMD, what
 // its registers allow), and the blocks are sized so that the waves spread evenly over all 256
@@ -1669,8 +1677,7 @@ ResidentShape resident_shape(uint32_t ntiles, uint32_t nunits, uint32_t rows, bo
         s.nw = std::max(per_cu, 4u);  // at least four waves to stage h
     s.blocks = (waves + s.nw - 1) / s.nw;
     s.bytes = bytes(s.nw);
-    // short streams, and more blocks than CUs, finish together
-    s.tree = s.rt == 1 || s.blocks > kCUs;
+    s.tree = finish_by_groups(s.rt, s.blocks, nunits);
     // RMSNorm rows run here wherever their two halves fit, five to eight rows too (V = 262,144, M = 5,
     // against the prep launch and the streamed-h kernel: d = 1,024 29.2 and 37.3 us, d = 2,560 62.2 and
     // 72.9, d = 5,376 124.8 and 134.9; seven rows of d = 5,376 no longer fit)
@@ -1740,7 +1747,7 @@ FinishEpochs finish_epochs(twd_head* h, bool tree) {
 template <int MODE>
 hipError_t launch_stream(twd_head* h, HeadArgs& a, hipStream_t stream) {
     const StreamShape s = stream_shape(h->ntiles);
-    a.ep = finish_epochs<MODE>(h, s.rt == 1 || s.blocks > kCUs);
+    a.ep = finish_epochs<MODE>(h, finish_by_groups(s.rt, s.blocks, h->nunits));
     auto go = [&](auto kernel) { kernel<<<s.blocks, s.nw * 64, 0, stream>>>(a, h->hp, h->hx); };
     if (s.rt == 1)
         go(head_stream_kernel<1, 4, MODE>);
