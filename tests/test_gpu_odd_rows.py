@@ -46,3 +46,20 @@ def test_rows_where_a_thread_takes_more_records(oracle, V, rows, k):
     sel.close()
     want = [oracle.sample_token(x[m], p.temperature, p.top_p, p.top_k, u=p.uniform) for m, p in enumerate(prm)]
     assert got.tolist() == want
+
+
+# both sides of the record words' line for many rows: shortlists of mean 128 and 256, and mixed ones
+@pytest.mark.parametrize("V,rows", [(32003, 9), (262144, 48)])
+@pytest.mark.parametrize("ks", [(127,), (128,), (256,), (40, 250, 1)])
+def test_many_rows_with_and_without_words(oracle, V, rows, ks):
+    import torch
+    t = twd()
+    rng = np.random.default_rng(V + rows + sum(ks))
+    x = (3.0 * rng.standard_normal((rows, V))).astype(np.float32)
+    prm = [t.RowParams(0.8, 0.97 if m % 2 else 1.0, ks[m % len(ks)], 1.0, float(np.float32(rng.uniform(0, 0.999))),
+                       0.0, 0, 0) for m in range(rows)]
+    sel = t.Selector(V, rows)
+    got = sel.select(torch.from_numpy(x).cuda(), prm).cpu().numpy().astype(np.int64) & 0xFFFFFFFF
+    sel.close()
+    want = [oracle.sample_token(x[m], p.temperature, p.top_p, p.top_k, u=p.uniform) for m, p in enumerate(prm)]
+    assert got.tolist() == want

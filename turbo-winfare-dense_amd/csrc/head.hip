@@ -1651,14 +1651,14 @@ bool finish_by_groups(int rt, uint32_t blocks, uint32_t nunits) {
 // CUs in one round: one block per CU up to 12 waves, two of half as many past that (a block's
 // staging and finish then overlap the other's stream) where two copies of h fit in LDS. With more
 // than four rows, staging is longer: exactly 16 waves are one block, and 13 to 15 one block of 16 on
-// fewer CUs past kHalvesChunks chunks (M = 5 greedy, halves and 16, us: V = 200,003 d = 1,024 22.7 and
-// 24.1, 2,048 40.9 and 41.6, 3,584 67.9 and 65.6; V = 230,000 d = 2,560, M = 8 55.0 and 53.8, d = 4,096
-// 86.2 and 83.4). Larger heads take further rounds of 8- or 16-wave blocks. Measured against four tiles per wave and 8- or
-// 16-wave blocks throughout (M = 1 / M = 5, greedy, us): V = 32,003 d = 2,048 (RT 1, 8 waves)
-// 19.2 -> 12.3 / 33.1 -> 13.7; V = 65,536 d = 4,096 (RT 1, 2 x 8 / 16) 36.6 -> 27.5 / 60.9 -> 29.7;
-// V = 100,003 d = 2,560 (RT 2, 2 x 7) 29.0 -> 27.1 / 42.7 -> 28.8; V = 151,669 d = 3,584 (RT 4,
-// 10) 64.3 -> 51.8 / 58.7 -> 53.8; V = 262,144 d = 5,376 unchanged. With the finish by groups and
-// h requested first, V = 32,003: 10.9 / 11.8.
+// fewer CUs past kHalvesChunks chunks (M = 5 greedy, halves and 16, us: V = 200,003 d = 1,024 22.7
+// and 24.1, 2,048 40.9 and 41.6, 3,584 67.9 and 65.6; V = 230,000 d = 2,560, M = 8 55.0 and 53.8,
+// d = 4,096 86.2 and 83.4). Larger heads take further rounds of 8- or 16-wave blocks. Measured
+// against four tiles per wave and 8- or 16-wave blocks throughout (M = 1 / M = 5, greedy, us):
+// V = 32,003 d = 2,048 (RT 1, 8 waves) 19.2 -> 12.3 / 33.1 -> 13.7; V = 65,536 d = 4,096 (RT 1, 2 x 8 /
+// 16) 36.6 -> 27.5 / 60.9 -> 29.7; V = 100,003 d = 2,560 (RT 2, 2 x 7) 29.0 -> 27.1 / 42.7 -> 28.8;
+// V = 151,669 d = 3,584 (RT 4, 10) 64.3 -> 51.8 / 58.7 -> 53.8; V = 262,144 d = 5,376 unchanged. With
+// the finish by groups and h requested first, V = 32,003: 10.9 / 11.8.
 constexpr uint32_t kHalvesChunks = 16;
 
 struct ResidentShape {

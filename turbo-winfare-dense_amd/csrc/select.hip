@@ -1570,10 +1570,21 @@ void wave_stats_kernel(WaveStatsBufs b) {
 }
 
 // When the record pass also forms the record words: for few rows, whose blocks are short of work,
-// and for long shortlists, whose merges they spare the most gathering (48 rows of V = 262,144, us:
-// k = 0 33.4 -> 30.8, k = 150 28.5 -> 28.0, but k = 64 24.4 -> 26.3).
+// and for long shortlists, whose merges they spare the most gathering. The words cost the pass time by
+// the entries of all rows, and a merge is spared time by its own shortlist (from 128 entries on, where it
+// gathers in more batches), so the mean shortlist past 64 is held against the entries. Without the words
+// and with them, us: 48 rows of V = 32,003 k = 128 15.9 and 15.9, k = 256 22.2 and 19.1; of 151,669 k = 128
+// 22.9 and 22.2, k = 256 28.2 and 25.2; of 262,144 k = 64 24.3 and 26.4, k = 128 27.4 and 27.7, k = 200 29.4 and 28.8;
+// 64 rows of 262,144 k = 128 30.8 and 31.7, k = 256 36.2 and 34.4; of 500,000 k = 128 46.7 and 49.6, k = 200
+// 48.5 and 50.7.
 constexpr uint32_t kAuxMaxRows = 8;
 constexpr uint32_t kAuxMeanWant = 128;
+
+static bool want_aux(uint32_t rows, uint32_t vocab, uint32_t want_sum) {
+    if (rows <= kAuxMaxRows) return true;
+    if (want_sum < kAuxMeanWant * rows) return false;
+    return static_cast<uint64_t>(rows) * rows * vocab <= 175000ull * (want_sum - 64ull * rows);
+}
 
 __global__ void verify_compare_kernel(const uint32_t* row_tokens, uint32_t rows,
                                       const uint32_t* drafts, uint32_t nd,
@@ -1985,7 +1996,7 @@ int launch_select(const SelectScratch& s, float* logits, uint32_t vocab, uint32_
             penalty_hash_kernel<<<rows, kPhThreads, 0, stream>>>(a, pb);
             TWD_HIP(hipGetLastError());
         }
-        const bool aux = any_short && (rows <= kAuxMaxRows || short_want >= kAuxMeanWant * rows);
+        const bool aux = any_short && want_aux(rows, vocab, short_want);
         const SampleStats st{s.wkey, s.wsum, s.wmax, aux ? s.waux : nullptr, __builtin_nanf("")};  // no cap
         WaveStatsBufs wb{logits, stride, vocab, waves, st};
         const dim3 grid((vocab + kWsEntries - 1) / kWsEntries, rows);
