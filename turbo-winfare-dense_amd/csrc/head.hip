@@ -244,53 +244,44 @@ __device__ __forceinline__ uint64_t row16_max_u64(uint64_t k) {
     return k;
 }
 
-template <int NMT, int NI, int RT, int MODE, int MS = 1, typename Epi>
-__device__ __forceinline__ void head_epilogue(const HeadArgs& a, f32x4_t (&tot)[RT][NMT],
+template <int RT, int MODE, int MS = 1, typename Epi>
+__device__ __forceinline__ void head_epilogue(const HeadArgs& a, f32x4_t (&tot)[RT][1],
                                               uint32_t tile0, Epi& se) {
-    static_assert(MS == 1 || (NMT == 1 && NI == 4), "spread rows live in one m tile");
-    if (NMT == 1 && a.fold) {  // rows r and r + 8 sit in lanes l and l + 32
+    if (a.fold) {  // rows r and r + 8 sit in lanes l and l + 32
 #pragma unroll
         for (int j = 0; j < RT; ++j)
 #pragma unroll
-            for (int i = 0; i < NI; ++i) tot[j][0][i] += __shfl_xor(tot[j][0][i], 32);
+            for (int i = 0; i < 4; ++i) tot[j][0][i] += __shfl_xor(tot[j][0][i], 32);
     }
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    uint64_t best[NMT][NI];
-#pragma unroll
-    for (int mt = 0; mt < NMT; ++mt)
-#pragma unroll
-        for (int i = 0; i < NI; ++i) best[mt][i] = 0;
+    uint64_t best[4] = {0, 0, 0, 0};
 
 #pragma unroll
     for (int j = 0; j < RT; ++j) {
         const uint32_t r = (tile0 + j) * kTileRows + (lane & 15);
 #pragma unroll
-        for (int mt = 0; mt < NMT; ++mt)
-#pragma unroll
-            for (int i = 0; i < NI; i += MS) {
-                const uint32_t m = (mt * 16 + 4 * (lane >> 4) + i) / MS;
-                float v = tot[j][mt][i];
-                if (a.softcap > 0.0f) v = a.softcap * tanhf(v / a.softcap);
-                const bool live = (m < a.M) && (r < a.vocab);
-                if (live && a.logits) a.logits[static_cast<size_t>(m) * a.vocab + r] = v;
-                if (MODE != kModeLogits) {
-                    const uint64_t k = live ? rank_key(v, r) : 0ull;
-                    best[mt][i] = k > best[mt][i] ? k : best[mt][i];
-                }
+        for (int i = 0; i < 4; i += MS) {
+            const uint32_t m = (4 * (lane >> 4) + i) / MS;
+            float v = tot[j][0][i];
+            if (a.softcap > 0.0f) v = a.softcap * tanhf(v / a.softcap);
+            const bool live = (m < a.M) && (r < a.vocab);
+            if (live && a.logits) a.logits[static_cast<size_t>(m) * a.vocab + r] = v;
+            if (MODE != kModeLogits) {
+                const uint64_t k = live ? rank_key(v, r) : 0ull;
+                best[i] = k > best[i] ? k : best[i];
             }
+        }
     }
     if (MODE == kModeLogits) return;
 
     // rows sharing m are the 16 lanes with the same lane >> 4, one DPP row (register moves, where a
     // shuffle is an LDS round trip at the end of every wave)
 #pragma unroll
-    for (int mt = 0; mt < NMT; ++mt)
-#pragma unroll
-        for (int i = 0; i < NI; i += MS) {
-            const uint64_t k = row16_max_u64(best[mt][i]);
-            const uint32_t m = (mt * 16 + 4 * (lane >> 4) + i) / MS;
-            if ((lane & 15) == 0 && m < static_cast<uint32_t>(Epi::kRows)) se.red[wave][m] = k;
-        }
+    for (int i = 0; i < 4; i += MS) {
+        const uint64_t k = row16_max_u64(best[i]);
+        const uint32_t m = (4 * (lane >> 4) + i) / MS;
+        if ((lane & 15) == 0 && m < static_cast<uint32_t>(Epi::kRows)) se.red[wave][m] = k;
+    }
     grid_finish(a, se);
 }
 
@@ -885,7 +876,7 @@ __global__ __launch_bounds__(kResidentWaves * 64) void head_small_kernel(HeadArg
     if constexpr (MODE == kModeSample) {
         head_epilogue_sample<RT, MS>(a, tot, tile0, block_row0, cnt, exp2_tbl, prm);
     } else {
-        head_epilogue<1, 4, RT, MODE, MS>(a, tot, tile0, se);
+        head_epilogue<RT, MODE, MS>(a, tot, tile0, se);
     }
 }
 
@@ -893,14 +884,13 @@ __global__ __launch_bounds__(kResidentWaves * 64) void head_small_kernel(HeadArg
 // call and streamed through LDS; M > 16 runs head_wide32_kernel below
 //
 // prep_hidden_kernel writes, once per call, the prepared h in A-fragment order,
-// hp[U][mt][t][lane] (16 B each, rows m >= M zero), and the bias A-fragment entries
-// hx[P][mt][lane] of super-unit P (groups past the end zero).
-template <int NMT>
+// hp[U][t][lane] (16 B each, rows m >= M zero), and the bias A-fragment entries
+// hx[P][lane] of super-unit P (groups past the end zero).
 __global__ __launch_bounds__(kHeadThreads) void prep_hidden_kernel(const uint16_t* __restrict__ h,
                                                                    uint32_t M, uint32_t d,
                                                                    u32x4_t* __restrict__ hp,
                                                                    u32x4_t* __restrict__ hx) {
-    const uint32_t per_chunk = NMT * 256;  // 16 B vectors per chunk (NMT*16 rows x 16)
+    constexpr uint32_t per_chunk = 256;  // 16 B vectors per chunk (16 rows x 16)
     const uint32_t nunits = d / kChunkK;
     // an odd chunk count is padded with one zero chunk: the kernel always computes both
     // chunks of a stage, and a zero h makes the padding add exactly nothing
@@ -916,14 +906,12 @@ __global__ __launch_bounds__(kHeadThreads) void prep_hidden_kernel(const uint16_
     s += __shfl_xor(s, 2);
     s += __shfl_xor(s, 4);
     if (U < padded) {
-        hp[((static_cast<size_t>(U) * NMT + (m >> 4)) * 4 + (c >> 2)) * 64 + (c & 3) * 16 + (m & 15)] =
-            prep_h(v);
+        hp[(static_cast<size_t>(U) * 4 + (c >> 2)) * 64 + (c & 3) * 16 + m] = prep_h(v);
         if ((c & 7) == 0) {
             const uint32_t g = 2 * U + (c >> 3);
             uint32_t* x = reinterpret_cast<uint32_t*>(hx);
             auto at = [&](int kg) {
-                return x + (((static_cast<size_t>(g >> 2) * NMT + (m >> 4)) * 4 + kg) * 16 + (m & 15)) * 4 +
-                       (g & 3);
+                return x + ((static_cast<size_t>(g >> 2) * 4 + kg) * 16 + m) * 4 + (g & 3);
             };
             bias_slices(s, at);  // zero slices for the padding chunk's two groups
         }
@@ -936,8 +924,8 @@ __global__ __launch_bounds__(kHeadThreads) void prep_hidden_kernel(const uint16_
 // it is split into h_hi = bf16(h) and h_lo = bf16(h - h_hi) (|h - h_hi - h_lo| <= 2^-18 |h|),
 // placed as MFMA rows m and m + 8 of one 16-row tile; the kernel's epilogue adds row m + 8 to
 // row m (HeadArgs::fold). The bias term of each row uses the group sums of its own half.
-// Every block recomputes the rows' mean squares itself (M x d fp32 from L2), so the prologue
-// needs no launch of its own. Output: the hp / hx layout of prep_hidden_kernel<1>.
+// Every block recomputes the rows' mean squares itself (M x d fp32 from L2), so they need no launch
+// before this one. Output: the hp / hx layout of prep_hidden_kernel.
 __global__ __launch_bounds__(kHeadThreads) void prep_rmsnorm_kernel(const float* __restrict__ x,
                                                                     const uint16_t* __restrict__ w,
                                                                     float eps, uint32_t M, uint32_t d,
@@ -1174,10 +1162,10 @@ void head_stream_kernel(HeadArgs a, const u32x4_t* __restrict__ hp, const u32x4_
             step(hc, xc, w * kWinChunks + c, std::integral_constant<int, k + 1>{}, std::false_type{});
         }
     });
-    head_epilogue<1, 4, RT, MODE>(a, tot, tile0, se);
+    head_epilogue<RT, MODE>(a, tot, tile0, se);
 }
 
-// ---- 33 <= M <= 64: 32x32x16 MFMAs, weights and h streamed into LDS two chunks ahead ----------
+// ---- 17 <= M <= 64: 32x32x16 MFMAs, weights and h streamed into LDS two chunks ahead ----------
 //
 // Lane l = 32 kh + n of a 32 x 32 x 16 MFMA carries B column n (a vocabulary row of the wave's
 // tile pair: tile n / 16, row n % 16) and k half kh. For k-step s of group g (64 columns) it
@@ -1892,8 +1880,7 @@ int launch_head(twd_head* h, const uint16_t* hidden, uint32_t rows, float* logit
         a.ep = finish_epochs<MODE>(h, shape.tree);
         TWD_HIP((launch_resident<MODE, false>(shape, a, stream)));
     } else if (rows <= kStreamRows) {
-        prep_hidden_kernel<1><<<padded_units(h->nunits) * 1, kHeadThreads, 0, stream>>>(hidden, rows, h->d,
-                                                                                       h->hp, h->hx);
+        prep_hidden_kernel<<<padded_units(h->nunits), kHeadThreads, 0, stream>>>(hidden, rows, h->d, h->hp, h->hx);
         TWD_HIP(launch_stream<MODE>(h, a, stream));
     } else if (rows <= 32) {
         a.ep = finish_epochs<MODE>(h, false);

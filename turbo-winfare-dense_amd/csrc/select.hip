@@ -421,14 +421,18 @@ __global__ __launch_bounds__(kSmThreads) void select_sample_merge_kernel(SelectA
 // one row, before (4 or 8 a thread) and after: V = 32,003 11.8 and 10.7 us, V = 100,003 10.6 and 9.9,
 // V = 262,144 (4 a thread either way) 11.5 and 11.2; 8 rows 12.2 and 11.1, 13.2 and 12.4, 13.6 and 13.5.
 using MergeKernel = void (*)(SelectArgs, SampleMergeBufs);
+// Records of 16 entries are at most 4,096 (one tile per wave), records of 32 from 2,049 to 4,096 (two):
+// counts outside those are no call's (null).
 template <uint32_t RSH>
 MergeKernel merge_kernel(uint32_t waves) {
-    if (waves <= kSmThreads) return select_sample_merge_kernel<RSH, 1>;
-    if (waves <= kSmThreads * 2) return select_sample_merge_kernel<RSH, 2>;
+    if constexpr (RSH != 5) {
+        if (waves <= kSmThreads) return select_sample_merge_kernel<RSH, 1>;
+        if (waves <= kSmThreads * 2) return select_sample_merge_kernel<RSH, 2>;
+    }
     if (waves <= kSmThreads * (kSmPer / 2)) return select_sample_merge_kernel<RSH, kSmPer / 2>;
-    return select_sample_merge_kernel<RSH, kSmPer>;
+    if constexpr (RSH == 6) return select_sample_merge_kernel<RSH, kSmPer>;
+    return nullptr;
 }
-
 
 // ---- shortlists longer than 256: top_k > 256 -------------------------------------------------------
 //
@@ -1913,7 +1917,7 @@ int enable_select_kernels() {
                                       static_cast<int>(sizeof(MergeShared)));
         for (uint32_t waves : {1u, kSmThreads + 1u, 2 * kSmThreads + 1u, kSampleMaxWaves})
             for (MergeKernel merge : {merge_kernel<4>(waves), merge_kernel<5>(waves), merge_kernel<6>(waves)})
-                if (err == hipSuccess)
+                if (err == hipSuccess && merge)
                     err = hipFuncSetAttribute(reinterpret_cast<const void*>(merge),
                                               hipFuncAttributeMaxDynamicSharedMemorySize,
                                               static_cast<int>(sizeof(SampleMergeShared)));
@@ -2074,13 +2078,12 @@ int launch_sample_merge(const SampleStats& st, uint32_t waves, uint32_t rec_rows
     b.st = st;
     b.tokens = tokens;
     b.mirror = mirror;
-    auto merge = [&](MergeKernel kernel) { kernel<<<rows, kSmThreads, sizeof(SampleMergeShared), stream>>>(a, b); };
-    switch (rec_rows) {
-        case 16: merge(merge_kernel<4>(waves)); break;
-        case 32: merge(merge_kernel<5>(waves)); break;
-        case 64: merge(merge_kernel<6>(waves)); break;
-        default: return fail(TWD_E_INVALID, "sample merge: record rows out of range");
-    }
+    const MergeKernel merge = rec_rows == 16   ? merge_kernel<4>(waves)
+                              : rec_rows == 32 ? merge_kernel<5>(waves)
+                              : rec_rows == 64 ? merge_kernel<6>(waves)
+                                               : nullptr;
+    if (!merge) return fail(TWD_E_INVALID, "sample merge: record rows out of range");
+    merge<<<rows, kSmThreads, sizeof(SampleMergeShared), stream>>>(a, b);
     TWD_HIP(hipGetLastError());
     return launch_long(lng, st, waves, rec_rows, logits, vocab, vocab, rows, params, tokens, stream);
 }
