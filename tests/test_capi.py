@@ -193,3 +193,27 @@ def test_generator_ex_argument_errors_without_gpu():
     assert lib.twd_generator_stop_reason(None) == t.twd.STOP_NONE
     lib.twd_generator_cancel(None)  # a no-op on a null generator
     assert lib.twd_head_finish_state(None) is None
+
+
+def test_draft_rows_are_checked_on_every_call(monkeypatch):
+    # a shorter or strided view at an address of the call before is refused
+    import torch
+    t = twd()
+    calls = []
+    monkeypatch.setattr(t.twd, "lib", type("Lib", (), {"twd_verify_draft": staticmethod(
+        lambda *a: calls.append(a) or 0)}))
+    sel = object.__new__(t.Selector)
+    sel.handle, sel._draft_ptrs = None, None
+    logits, row = torch.zeros(2, 64), torch.zeros(128)
+    result = torch.zeros(t.VERIFY_WORDS, dtype=torch.int32)
+    drafts = torch.zeros(1, dtype=torch.int32)
+    p = t.RowParams(0.8, 0.95, 4, 1.0, 0.0, 0.0, 0, 0)
+    for rows in ([row[:64]], [row[:64]], [None]):
+        sel.verify_draft(logits, rows, p, 1, drafts, result=result, stream=0)
+    assert len(calls) == 3
+    sel.verify_draft(logits, [row[:64]], p, 1, drafts, result=result, stream=0)
+    for bad in (row[:32], row[::2]):
+        assert bad.data_ptr() == row.data_ptr()
+        with pytest.raises(ValueError):
+            sel.verify_draft(logits, [bad], p, 1, drafts, result=result, stream=0)
+    assert len(calls) == 4

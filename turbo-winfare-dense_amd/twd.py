@@ -311,14 +311,14 @@ class Selector:
             result = torch.zeros(VERIFY_WORDS, dtype=torch.int32, device=logits.device)
         if logits.stride(1) != 1:
             raise ValueError("logit rows must be contiguous")
+        for r in draft_rows:
+            if r is not None and (r.numel() != vocab or not r.is_contiguous()):
+                raise ValueError("each draft row must be a contiguous row of vocab floats")
         # the pointer array of the last list of draft rows is kept, so repeated calls with the
         # same rows only compare their addresses
         key = tuple(0 if r is None else r.data_ptr() for r in draft_rows)
         cached = self._draft_ptrs
         if cached is None or cached[0] != key:
-            for r in draft_rows:
-                if r is not None and (r.numel() != vocab or not r.is_contiguous()):
-                    raise ValueError("each draft row must be a contiguous row of vocab floats")
             cached = (key, (_vp * max(1, len(key)))(*[k or None for k in key]))
             self._draft_ptrs = cached
         stride = logits.stride(0) if rows > 1 else vocab
