@@ -157,3 +157,28 @@ def test_small_vocabularies_taken_whole(env, oracle, V):
     rows.append(wide)
     params.append(t.RowParams(float("inf"), 1.0, min(V, 4096), 1.0, 0.8, 0.0, 0, 0))
     check(env, oracle, rows, params, V)
+
+
+@pytest.mark.ties
+@pytest.mark.parametrize("V", [50_000, 100_000, 140_001])
+def test_overfull_lists_from_the_fused_pass(env, oracle, V):
+    # records of 16, 32 and 64 entries; weights of few rows differ from zero, so nearly all logits are equal
+    torch, dev, t, _ = env
+    d = 128
+    W = np.zeros((V, d // 8), np.uint32)
+    S = np.full((V, d // 64), 0x3F80, np.uint16)  # 1.0
+    B = np.zeros((V, d // 64), np.uint16)
+    rng = np.random.default_rng(V)
+    some = rng.choice(V, 40, replace=False)
+    W[some] = rng.integers(0, 2 ** 32, (40, d // 8), dtype=np.uint64).astype(np.uint32)
+    wsb = np.concatenate([W.reshape(-1).view(np.uint8), S.reshape(-1).view(np.uint8), B.reshape(-1).view(np.uint8)])
+    head = t.LMHead(torch.from_numpy(wsb).to(dev), V, d, 30.0)
+    bits = np.full((3, d), 0x3C00, np.uint16)  # 2^-7
+    bits[1] = 0xBC00  # -2^-7: the 40 rows lie below the others
+    h = torch.from_numpy(bits.view(np.int16)).to(dev)
+    prm = [t.RowParams(0.9, 0.97, k, 1.0, u, 30.0, 0, 0) for k, u in ((300, 0.7), (1000, 0.31), (4096, 0.999))]
+    tok, lg = head.sample(h, prm)
+    tok, lg = tok.cpu().numpy(), lg.cpu().numpy()
+    for m, p in enumerate(prm):
+        assert int(tok[m]) & 0xFFFFFFFF == oracle.sample_token(lg[m], p.temperature, p.top_p, p.top_k, u=p.uniform)
+    head.close()
