@@ -1587,7 +1587,7 @@ constexpr uint32_t kAuxMeanWant = 128;
 static bool want_aux(uint32_t rows, uint32_t vocab, uint32_t want_sum) {
     if (rows <= kAuxMaxRows) return true;
     if (want_sum < kAuxMeanWant * rows) return false;
-    return static_cast<uint64_t>(rows) * rows * vocab <= 175000ull * (want_sum - 64ull * rows);
+    return static_cast<uint64_t>(rows) * rows * vocab <= 160000ull * (want_sum - 64ull * rows);
 }
 
 __global__ void verify_compare_kernel(const uint32_t* row_tokens, uint32_t rows,
